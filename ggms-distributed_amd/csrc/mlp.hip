@@ -11,11 +11,11 @@
 //
 // Parameter layout (row-major fp32): W1[32][65], b1[32], W2[32], b2.
 //
-// Kernels: batched forward; loss + gradient in two steps (per-sample
-// back-propagation to the hidden layer, then one thread per parameter summing
-// over a chunk of samples); an Adam step.
+// Kernels: batched forward; loss + gradient in two steps (per workgroup over
+// its tiles of samples, then the sum of the workgroups' partials); an Adam step.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -39,96 +39,218 @@ const float* learned_weights_device(int device) {
 
 __device__ __forceinline__ float sigmoidf_(float o) { return 1.0f / (1.0f + __expf(-o)); }
 
-__global__ void __launch_bounds__(256) k_mlp_forward(const float* __restrict__ w, const float* __restrict__ x,
-                                                     uint32_t nb, float* __restrict__ out) {
-  __shared__ float sw[MP];
-  for (int i = threadIdx.x; i < MP; i += blockDim.x) sw[i] = w[i];
-  __syncthreads();
-  uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
-  const float* xb = x + (size_t)b * MI;
-  float in[MI];
-  for (int i = 0; i < MI; ++i) in[i] = xb[i];
-  const float* W1 = sw;
-  const float* b1 = sw + MH * MI;
-  const float* W2 = b1 + MH;
-  float o = W2[MH];
-  for (int h = 0; h < MH; ++h) {
-    float z = b1[h];
-    for (int i = 0; i < MI; ++i) z += W1[h * MI + i] * in[i];
-    o += W2[h] * fmaxf(z, 0.0f);
+// One 64-sample tile per step and workgroup, four waves.  The products run on
+// the fp32 matrix cores (16x16x4): a sample's hidden layer is one row of
+// X [64 x 68] * W1^T [68 x 32], column 65 of X being 1 and of W1 the bias.
+constexpr uint32_t kTile = 64, kMlpThreads = 256;
+// row strides in LDS: 68 = 4 mod 32 spreads the operands' 16 rows x 4 columns
+// over every bank; 48 does the same for the 4 rows x 16 columns of dz
+constexpr uint32_t kXStride = 68, kZStride = 48;
+constexpr uint32_t kMaxGradWgs = 256;
+constexpr uint32_t kPart = MP + 1;  // floats of one workgroup's partial: gradient, loss
+
+using f32x4 = float __attribute__((ext_vector_type(4)));
+
+struct MlpLds {
+  float x[kTile * kXStride + 16];  // + 16: the last column tile reads past the last row (columns not used)
+  float w1[MH * kXStride];
+  float w2[MH + 1];
+};
+
+__device__ __forceinline__ void mlp_load_weights(MlpLds& L, const float* __restrict__ w) {
+  for (uint32_t j = threadIdx.x; j < MH * kXStride; j += kMlpThreads) {
+    const uint32_t h = j / kXStride, i = j % kXStride;
+    L.w1[j] = i < (uint32_t)MI ? w[h * MI + i] : i == (uint32_t)MI ? w[MH * MI + h] : 0.0f;
   }
-  out[b] = sigmoidf_(o);
+  if (threadIdx.x <= (uint32_t)MH) L.w2[threadIdx.x] = w[MH * MI + MH + threadIdx.x];
+  if (threadIdx.x < 16) L.x[kTile * kXStride + threadIdx.x] = 0.0f;
 }
 
-// Backward, step 1 (one thread per sample): forward pass, then the per-sample
-// quantities the weight gradient needs: dz[b][h] = dL/dz_h (zero where the
-// ReLU is off), a[b][h] = relu(z_h), d_o[b] = dL/do.  Loss is the mean of
-// 0.5 (sigmoid(o) - y)^2 over the batch.
-__global__ void __launch_bounds__(256) k_mlp_backprop(const float* __restrict__ w, const float* __restrict__ x,
-                                                      const float* __restrict__ y, uint32_t nb,
-                                                      float* __restrict__ dz, float* __restrict__ act,
-                                                      float* __restrict__ d_out, float* __restrict__ loss) {
-  __shared__ float sw[MP];
-  __shared__ float sl;
-  for (int i = threadIdx.x; i < MP; i += blockDim.x) sw[i] = w[i];
-  if (threadIdx.x == 0) sl = 0.0f;
-  __syncthreads();
-  uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nb) {
-    const float* xb = x + (size_t)b * MI;
-    float in[MI];
-    for (int i = 0; i < MI; ++i) in[i] = xb[i];
-    const float* W1 = sw;
-    const float* b1 = sw + MH * MI;
-    const float* W2 = b1 + MH;
-    float z[MH];
-    float o = W2[MH];
-    for (int h = 0; h < MH; ++h) {
-      float s = b1[h];
-      for (int i = 0; i < MI; ++i) s += W1[h * MI + i] * in[i];
-      z[h] = s;
-      o += W2[h] * fmaxf(s, 0.0f);
-    }
-    float p = sigmoidf_(o);
-    float e = p - y[b];
-    atomicAdd(&sl, 0.5f * e * e / (float)nb);
-    float d_o = e * p * (1.0f - p) / (float)nb;
-    d_out[b] = d_o;
-    for (int h = 0; h < MH; ++h) {
-      act[(size_t)b * MH + h] = fmaxf(z[h], 0.0f);
-      dz[(size_t)b * MH + h] = z[h] > 0.0f ? d_o * W2[h] : 0.0f;
-    }
+// Rows past nb are zero (their samples take no part).
+__device__ __forceinline__ void mlp_load_tile(MlpLds& L, const float* __restrict__ x, uint32_t b0, uint32_t nb) {
+  const uint32_t rows = nb - b0 < kTile ? nb - b0 : kTile;
+  const float* src = x + (size_t)b0 * MI;
+  for (uint32_t j = threadIdx.x; j < kTile * MI; j += kMlpThreads)
+    L.x[(j / MI) * kXStride + j % MI] = j < rows * MI ? src[j] : 0.0f;
+  if (threadIdx.x < kTile) {
+    float* r = L.x + threadIdx.x * kXStride + MI;
+    r[0] = 1.0f;
+    r[1] = 0.0f;
+    r[2] = 0.0f;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, sl);
 }
 
-// Backward, step 2 (one thread per parameter, one workgroup row per chunk of
-// samples): grad_W1 = sum_b dz_b x_b^T, grad_b1 = sum_b dz_b,
-// grad_W2 = sum_b d_o_b a_b, grad_b2 = sum_b d_o_b.
-constexpr uint32_t kGradChunk = 1024;
-__global__ void __launch_bounds__(256) k_mlp_wgrad(const float* __restrict__ x, const float* __restrict__ dz,
-                                                   const float* __restrict__ act, const float* __restrict__ d_out,
-                                                   uint32_t nb, float* __restrict__ grad) {
-  uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= (uint32_t)MP) return;
-  uint32_t b0 = blockIdx.y * kGradChunk;
-  uint32_t b1 = b0 + kGradChunk < nb ? b0 + kGradChunk : nb;
-  float acc = 0.0f;
-  if (p < (uint32_t)(MH * MI)) {
-    uint32_t h = p / MI, i = p % MI;
-    for (uint32_t b = b0; b < b1; ++b) acc += dz[(size_t)b * MH + h] * x[(size_t)b * MI + i];
-  } else if (p < (uint32_t)(MH * MI + MH)) {
-    uint32_t h = p - MH * MI;
-    for (uint32_t b = b0; b < b1; ++b) acc += dz[(size_t)b * MH + h];
-  } else if (p < (uint32_t)(MH * MI + 2 * MH)) {
-    uint32_t h = p - MH * MI - MH;
-    for (uint32_t b = b0; b < b1; ++b) acc += d_out[b] * act[(size_t)b * MH + h];
-  } else {
-    for (uint32_t b = b0; b < b1; ++b) acc += d_out[b];
+// The hidden layer of this wave's 16 samples: lane l holds, for hidden units
+// l % 16 (z[0]) and 16 + l % 16 (z[1]), samples 4 * (l / 16) + r.  o[r] is the
+// output before the sigmoid of those samples, in every lane of the group of 16.
+__device__ __forceinline__ void mlp_tile_forward(const MlpLds& L, f32x4 (&z)[2], float (&o)[4]) {
+  const uint32_t l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const float* xr = L.x + (wv * 16 + (l & 15)) * kXStride + (l >> 4);
+  const float* wr = L.w1 + (l & 15) * kXStride + (l >> 4);
+  z[0] = f32x4{0, 0, 0, 0};
+  z[1] = f32x4{0, 0, 0, 0};
+#pragma unroll
+  for (uint32_t s = 0; s < kXStride / 4; ++s) {
+    const float a = xr[4 * s];
+    z[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, wr[4 * s], z[0], 0, 0, 0);
+    z[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, wr[16 * kXStride + 4 * s], z[1], 0, 0, 0);
   }
-  atomicAdd(&grad[p], acc);
+  const float v0 = L.w2[l & 15], v1 = L.w2[16 + (l & 15)];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float c = v0 * fmaxf(z[0][r], 0.0f) + v1 * fmaxf(z[1][r], 0.0f);
+#pragma unroll
+    for (int d = 8; d > 0; d >>= 1) c += __shfl_xor(c, d, 16);
+    o[r] = c + L.w2[MH];
+  }
+}
+
+__global__ void __launch_bounds__(kMlpThreads) k_mlp_forward(const float* __restrict__ w, const float* __restrict__ x,
+                                                             uint32_t nb, float* __restrict__ out) {
+  __shared__ MlpLds L;
+  const uint32_t b0 = blockIdx.x * kTile;
+  mlp_load_weights(L, w);
+  mlp_load_tile(L, x, b0, nb);
+  __syncthreads();
+  f32x4 z[2];
+  float o[4];
+  mlp_tile_forward(L, z, o);
+  const uint32_t l = threadIdx.x & 63, m = (threadIdx.x >> 6) * 16 + 4 * (l >> 4);
+#pragma unroll
+  for (uint32_t r = 0; r < 4; ++r)
+    if ((l & 15) == r && b0 + m + r < nb) out[b0 + m + r] = sigmoidf_(o[r]);
+}
+
+// Loss and gradient of the tiles t = blockIdx.x, + gridDim.x, ...: the forward
+// pass, dL/dz of the tile into LDS, then grad[W1 | b1] = dz^T [32 x 64] * X
+// [64 x 66] as ten 16 x 16 products over the four waves (b1's column is X's
+// column of ones); the last wave adds W2, b2 and the loss.  The sums stay in
+// registers over the tiles and are written once: part[blockIdx.x], or the
+// gradient itself when one workgroup does it all.  Bound by latency: at 4096
+// samples 64 CUs hold one tile each (loads, two short chains of matrix
+// products, four barriers), 11.6 us, and the sum of the partials 4.0 us.  A
+// thread per sample and then a thread per parameter walking 1024 samples took
+// 20.5 + 334 us, and its sums (one chain of 1024) were less exact.
+__global__ void __launch_bounds__(kMlpThreads) k_mlp_grad(const float* __restrict__ w, const float* __restrict__ x,
+                                                          const float* __restrict__ y, uint32_t nb,
+                                                          float* __restrict__ part, float* __restrict__ grad,
+                                                          float* __restrict__ loss) {
+  __shared__ MlpLds L;
+  __shared__ float dz[kTile * kZStride], act[kTile * kZStride], d_o[kTile], e2[kTile];
+  const uint32_t l = threadIdx.x & 63, wv = threadIdx.x >> 6, c16 = l & 15, q = l >> 4;
+  mlp_load_weights(L, w);
+  // ten output tiles (two of hidden units x five of inputs): waves 0 and 1 take three, 2 and 3 two
+  const uint32_t first = wv < 2 ? 3 * wv : 6 + 2 * (wv - 2), mine = wv < 2 ? 3u : 2u;
+  f32x4 acc[3] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+  float g2 = 0.0f, gb = 0.0f, ls = 0.0f;  // the last wave's: W2 gradient (half the samples per lane), b2 gradient, loss
+  const uint32_t tiles = (nb + kTile - 1) / kTile;
+  for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const uint32_t b0 = t * kTile;
+    __syncthreads();  // the previous tile's rows are read
+    mlp_load_tile(L, x, b0, nb);
+    float yv[4];
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+      const uint32_t b = b0 + wv * 16 + 4 * q + r;
+      yv[r] = b < nb ? y[b] : 0.0f;
+    }
+    __syncthreads();
+    f32x4 z[2];
+    float o[4];
+    mlp_tile_forward(L, z, o);
+    const float v0 = L.w2[c16], v1 = L.w2[16 + c16];
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+      const uint32_t m = wv * 16 + 4 * q + r;
+      const float p = sigmoidf_(o[r]);
+      const float e = p - yv[r];
+      const bool in = b0 + m < nb;
+      const float d = in ? e * p * (1.0f - p) / (float)nb : 0.0f;
+      float* zr = dz + m * kZStride + c16;
+      float* ar = act + m * kZStride + c16;
+      zr[0] = z[0][r] > 0.0f ? d * v0 : 0.0f;
+      zr[16] = z[1][r] > 0.0f ? d * v1 : 0.0f;
+      ar[0] = fmaxf(z[0][r], 0.0f);
+      ar[16] = fmaxf(z[1][r], 0.0f);
+      if (c16 == r) {
+        d_o[m] = d;
+        e2[m] = in ? 0.5f * e * e / (float)nb : 0.0f;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < 3; ++j) {
+      if (j >= mine) break;
+      const uint32_t ot = first + j;
+      const float* zc = dz + q * kZStride + (ot / 5) * 16 + c16;
+      const float* xc = L.x + q * kXStride + (ot % 5) * 16 + c16;
+#pragma unroll
+      for (uint32_t s = 0; s < kTile / 4; ++s)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(zc[4 * s * kZStride], xc[4 * s * kXStride], acc[j], 0, 0, 0);
+    }
+    if (wv == 3) {
+      float a = 0.0f;
+      const uint32_t h = l & 31, m0 = (l >> 5) * (kTile / 2);
+#pragma unroll 8
+      for (uint32_t m = m0; m < m0 + kTile / 2; ++m) a += d_o[m] * act[m * kZStride + h];
+      g2 += a;
+      gb += d_o[l];
+      ls += e2[l];
+    }
+  }
+  float* dst = gridDim.x == 1 ? grad : part + (size_t)blockIdx.x * kPart;
+#pragma unroll
+  for (uint32_t j = 0; j < 3; ++j) {
+    if (j >= mine) break;
+    const uint32_t ot = first + j, i = (ot % 5) * 16 + c16;
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+      const uint32_t h = (ot / 5) * 16 + 4 * q + r;
+      if (i < (uint32_t)MI) dst[h * MI + i] = acc[j][r];
+      else if (i == (uint32_t)MI) dst[MH * MI + h] = acc[j][r];
+    }
+  }
+  if (wv == 3) {
+    g2 += __shfl_xor(g2, 32, 64);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      gb += __shfl_xor(gb, d, 64);
+      ls += __shfl_xor(ls, d, 64);
+    }
+    if (l < (uint32_t)MH) dst[MH * MI + MH + l] = g2;
+    if (l == 0) {
+      dst[MP - 1] = gb;
+      if (gridDim.x == 1) *loss = ls;
+      else dst[MP] = ls;
+    }
+  }
+}
+
+// Sums the workgroups' partials in their order: 64 columns a workgroup, four
+// waves taking every fourth partial, eight reads in flight.
+__global__ void __launch_bounds__(256) k_mlp_sum(const float* __restrict__ part, uint32_t parts,
+                                                 float* __restrict__ grad, float* __restrict__ loss) {
+  __shared__ float s[4][64];
+  const uint32_t l = threadIdx.x & 63, wv = threadIdx.x >> 6, c = blockIdx.x * 64 + l;
+  float a = 0.0f;
+  if (c < kPart) {
+    uint32_t g = wv;
+    for (; g + 28 < parts; g += 32) {
+      float v[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) v[u] = part[(size_t)(g + 4 * u) * kPart + c];
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) a += v[u];
+    }
+    for (; g < parts; g += 4) a += part[(size_t)g * kPart + c];
+  }
+  s[wv][l] = a;
+  __syncthreads();
+  if (wv == 0 && c < kPart) {
+    const float t = (s[0][l] + s[1][l]) + (s[2][l] + s[3][l]);
+    if (c < (uint32_t)MP) grad[c] = t;
+    else *loss = t;
+  }
 }
 
 __global__ void k_fill_f32(float* __restrict__ p, uint32_t n, float v) {
@@ -191,7 +313,7 @@ ggms_status ggms_clear_learned_weights(int device) {
 ggms_status ggms_mlp_forward(const float* d_w, const float* d_x, uint32_t nb, float* d_out, void* stream) {
   if (!d_w || (!d_x && nb) || (!d_out && nb)) return GGMS_EINVAL;
   if (nb == 0) return GGMS_OK;
-  k_mlp_forward<<<(nb + 255) / 256, 256, 0, (hipStream_t)stream>>>(d_w, d_x, nb, d_out);
+  k_mlp_forward<<<(nb - 1) / kTile + 1, kMlpThreads, 0, (hipStream_t)stream>>>(d_w, d_x, nb, d_out);
   return hipGetLastError() == hipSuccess ? GGMS_OK : GGMS_EDEVICE;
 }
 
@@ -201,15 +323,16 @@ ggms_status ggms_mlp_loss_grad(const float* d_w, const float* d_x, const float* 
                                float* d_loss, float* d_work, void* stream) {
   if (!d_w || !d_grad || !d_loss || (nb && (!d_x || !d_y || !d_work))) return GGMS_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  k_fill_f32<<<(MP + 255) / 256, 256, 0, st>>>(d_grad, MP, 0.0f);
-  k_fill_f32<<<1, 32, 0, st>>>(d_loss, 1, 0.0f);
-  if (nb) {
-    float* dz = d_work;
-    float* act = d_work + (size_t)nb * MH;
-    float* dout = act + (size_t)nb * MH;
-    k_mlp_backprop<<<(nb + 255) / 256, 256, 0, st>>>(d_w, d_x, d_y, nb, dz, act, dout, d_loss);
-    dim3 g((MP + 255) / 256, (nb + kGradChunk - 1) / kGradChunk);
-    k_mlp_wgrad<<<g, 256, 0, st>>>(d_x, dz, act, dout, nb, d_grad);
+  if (!nb) {
+    k_fill_f32<<<(MP + 255) / 256, 256, 0, st>>>(d_grad, MP, 0.0f);
+    k_fill_f32<<<1, 32, 0, st>>>(d_loss, 1, 0.0f);
+  } else {
+    // a workgroup per tile up to one per CU, and no more than the workspace
+    // (2 MH + 1 floats a sample) holds partials of; a single one writes the result
+    uint64_t wgs = std::min<uint64_t>((nb - 1) / kTile + 1, ggms_mlp_workspace_floats(nb) / kPart);
+    wgs = std::max<uint64_t>(1, std::min<uint64_t>(wgs, kMaxGradWgs));
+    k_mlp_grad<<<(uint32_t)wgs, kMlpThreads, 0, st>>>(d_w, d_x, d_y, nb, d_work, d_grad, d_loss);
+    if (wgs > 1) k_mlp_sum<<<(kPart + 63) / 64, 256, 0, st>>>(d_work, (uint32_t)wgs, d_grad, d_loss);
   }
   return hipGetLastError() == hipSuccess ? GGMS_OK : GGMS_EDEVICE;
 }
