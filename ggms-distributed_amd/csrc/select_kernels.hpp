@@ -110,13 +110,15 @@ struct Plan0Args {
 // ---------------------------------------------------------------------------
 // workgroup utilities
 // ---------------------------------------------------------------------------
+// Inclusive scan over the wave (every lane active) in six DPP adds: by 1, 2, 4
+// and 8 inside each row of 16 lanes, then each row's total into the rows above.
 __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
-  const uint32_t lane = lane_id();
-#pragma unroll
-  for (uint32_t d = 1; d < 64; d <<= 1) {
-    uint32_t t = __shfl_up(v, d, 64);
-    if (lane >= d) v += t;
-  }
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
   return v;
 }
 
@@ -169,22 +171,20 @@ __device__ K wave_radix_select(const K* __restrict__ a, uint32_t len, K klo, K k
   return pre;
 }
 
-// Exclusive scan of one value per thread over the whole workgroup.
-// scratch: >= 16 u32 of LDS.  Returns exclusive prefix, total in *total.
+// Exclusive scan of one value per thread over the whole workgroup: a scan in
+// each wave, then every wave scans the waves' totals itself (lane w holds
+// wave w's).  scratch: >= 16 u32 of LDS.  Returns exclusive prefix, total in
+// *total.
 __device__ __forceinline__ uint32_t block_excl_scan_u32(uint32_t v, uint32_t* scratch, uint32_t* total) {
   const uint32_t lane = lane_id(), wv = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   uint32_t inc = wave_incl_scan_u32(v);
   __syncthreads();
   if (lane == 63) scratch[wv] = inc;
   __syncthreads();
-  uint32_t off = 0, tot = 0;
-  for (uint32_t w = 0; w < nw; ++w) {
-    uint32_t s = scratch[w];
-    if (w < wv) off += s;
-    tot += s;
-  }
-  *total = tot;
-  return off + inc - v;
+  const uint32_t mine = lane < nw ? scratch[lane] : 0u;
+  const uint32_t ws = wave_incl_scan_u32(mine);
+  *total = readlane_u32(ws, 63);
+  return readlane_u32(ws - mine, wv) + inc - v;
 }
 
 // Four exclusive scans at once (one pair of barriers instead of four).
@@ -198,24 +198,16 @@ __device__ __forceinline__ void block_excl_scan_u32x4(const uint32_t (&v)[4], ui
   __syncthreads();
   if (lane == 63) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) scratch[wv * 4 + i] = inc[i];
+    for (int i = 0; i < 4; ++i) scratch[i * 16 + wv] = inc[i];
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    off[i] = 0;
-    tot[i] = 0;
+    const uint32_t mine = lane < nw ? scratch[i * 16 + lane] : 0u;
+    const uint32_t ws = wave_incl_scan_u32(mine);
+    tot[i] = readlane_u32(ws, 63);
+    off[i] = readlane_u32(ws - mine, wv) + inc[i] - v[i];
   }
-  for (uint32_t w = 0; w < nw; ++w) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t s = scratch[w * 4 + i];
-      if (w < wv) off[i] += s;
-      tot[i] += s;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) off[i] += inc[i] - v[i];
 }
 
 // In-place inclusive scan of an LDS array of length L.  scratch >= 16 u32.
@@ -380,68 +372,195 @@ __device__ void bitonic_sort_lds_reg(K* s, uint32_t M) {
   }
 }
 
-// Key exchange with lane (lane ^ j) of the same wave (j < 64).
-template <class K>
-__device__ __forceinline__ K shfl_xor_key(K v, int j) {
+// Key of lane (lane ^ J) of the same wave, every lane active.  Inside a row of
+// 16 lanes it is one or two DPP moves; lanes 16 and 32 apart swap whole rows
+// (the permlane swaps).  No LDS access, unlike the general shuffle.
+template <int J>
+__device__ __forceinline__ uint32_t lane_xor_u32(uint32_t v) {
+#if defined(__AMDGCN__)
+  constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadXor3 = 0x1B, kHalfMirror = 0x141, kMirror = 0x140,
+                kRor8 = 0x128;
+  if constexpr (J == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kQuadXor1, 0xF, 0xF, true);
+  else if constexpr (J == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kQuadXor2, 0xF, 0xF, true);
+  else if constexpr (J == 3) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kQuadXor3, 0xF, 0xF, true);
+  else if constexpr (J == 4) return lane_xor_u32<3>(lane_xor_u32<7>(v));
+  else if constexpr (J == 7) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kHalfMirror, 0xF, 0xF, true);
+  else if constexpr (J == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kRor8, 0xF, 0xF, true);
+  else if constexpr (J == 15) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kMirror, 0xF, 0xF, true);
+  else if constexpr (J == 16) {  // both operands v: {value of the pair's lower row, of its upper row}
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return lane_id() & 16u ? r[0] : r[1];
+  } else if constexpr (J == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return lane_id() & 32u ? r[0] : r[1];
+  } else if constexpr (J == 31) return lane_xor_u32<16>(lane_xor_u32<15>(v));
+  else {
+    static_assert(J == 63, "lane_xor_u32");
+    return lane_xor_u32<32>(lane_xor_u32<31>(v));
+  }
+#else
+  return (uint32_t)__shfl_xor((int)v, J, 64);
+#endif
+}
+template <int J, class K>
+__device__ __forceinline__ K lane_xor_key(K v) {
   if constexpr (sizeof(K) == 8) {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, j, 64);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), j, 64);
+    const uint32_t lo = lane_xor_u32<J>((uint32_t)v), hi = lane_xor_u32<J>((uint32_t)(v >> 32));
     return ((K)hi << 32) | (K)lo;
   } else {
-    return (K)(uint32_t)__shfl_xor((int)(uint32_t)v, j, 64);
+    return (K)lane_xor_u32<J>((uint32_t)v);
+  }
+}
+
+// The lower (bound 0) or the upper (bound the largest key) key of a pair: the
+// median of the two and the bound, one v_med3_u32 for 32-bit keys.
+template <class K> __device__ __forceinline__ K pair_bound(bool keep_min) { return keep_min ? (K)0 : (K)~(K)0; }
+template <class K> __device__ __forceinline__ K pair_keep(K a, K b, K bound) {
+  const K lo = a < b ? a : b, hi = a < b ? b : a;
+  if constexpr (sizeof(K) == 4) {
+    const K m = hi < bound ? hi : bound;
+    return lo < m ? m : lo;
+  } else {
+    return bound ? hi : lo;
+  }
+}
+// Registers [0, E): the compare-exchanges at distances from, from / 2, .., 1,
+// all ascending; FLIP first pairs i with (2 from - 1 - i) inside every block.
+template <class K, int E, int FROM, bool FLIP>
+__device__ __forceinline__ void merge_regs(K (&r)[E]) {
+#pragma unroll
+  for (int st = FROM; st > 0; st >>= 1) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      if ((i & st) == 0) {
+        const int j = FLIP && st == FROM ? (i & ~(2 * FROM - 1)) + (2 * FROM - 1 - (i & (2 * FROM - 1))) : i + st;
+        const K lo = r[i] < r[j] ? r[i] : r[j], hi = r[i] < r[j] ? r[j] : r[i];
+        r[i] = lo;
+        r[j] = hi;
+      }
+    }
+  }
+}
+template <class K, int E, int SIZE = 2>
+__device__ __forceinline__ void sort_regs(K (&r)[E]) {
+  if constexpr (SIZE <= E) {
+    merge_regs<K, E, SIZE / 2, true>(r);
+    sort_regs<K, E, SIZE * 2>(r);
+  }
+}
+// The key the lane keeps of its own and lane (lane ^ J)'s.  The row swaps give
+// both keys of the pair to both lanes, which need not tell them apart.
+template <int J, class K>
+__device__ __forceinline__ K lane_pair(K v, K bound) {
+#if defined(__AMDGCN__)
+  if constexpr ((J == 16 || J == 32) && sizeof(K) == 4) {
+    if constexpr (J == 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      return pair_keep<K>(r[0], r[1], bound);
+    } else {
+      const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      return pair_keep<K>(r[0], r[1], bound);
+    }
+  }
+#endif
+  return pair_keep<K>(v, lane_xor_key<J, K>(v), bound);
+}
+// Lane stages at distances J, J / 2, .., 1 lanes, then the register stages.
+template <class K, int E, int J>
+__device__ __forceinline__ void merge_lanes(K (&r)[E]) {
+  if constexpr (J > 0) {
+    const K bound = pair_bound<K>((lane_id() & (uint32_t)J) == 0);
+#pragma unroll
+    for (int i = 0; i < E; ++i) r[i] = lane_pair<J, K>(r[i], bound);
+    merge_lanes<K, E, J / 2>(r);
+  } else {
+    merge_regs<K, E, E / 2, false>(r);
+  }
+}
+// Sorted runs of LANES / 2 lanes into sorted runs of LANES, up to a whole wave.
+template <class K, int E, int LANES = 2>
+__device__ __forceinline__ void sort_lanes(K (&r)[E]) {
+  if constexpr (LANES <= 64) {
+    const K bound = pair_bound<K>((lane_id() & (uint32_t)(LANES / 2)) == 0);
+    K p[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) p[i] = lane_xor_key<LANES - 1, K>(r[E - 1 - i]);
+#pragma unroll
+    for (int i = 0; i < E; ++i) r[i] = pair_keep<K>(r[i], p[i], bound);
+    merge_lanes<K, E, LANES / 4>(r);
+    sort_lanes<K, E, LANES * 2>(r);
   }
 }
 
 // Bitonic sort with the keys in registers throughout: thread t holds keys
 // [t*E, t*E + E) of M = E * T, T = M / E owning threads (a multiple of 64).  A
-// compare-exchange at distance d pairs thread t with t ^ (d / E): d < E stays
-// in registers, d / E < 64 is a lane shuffle inside the wave (no barrier),
-// and only d >= 64 E goes through LDS (own keys out, partner's keys in, two
-// barriers).  For M = 8192, E = 8 that is 10 barrier stages instead of 55.
+// merge first pairs key i of a block with its mirror image, so every
+// compare-exchange is ascending and which key a lane keeps depends on one bit
+// of its number.  Distances below E stay in registers, below 64 E they are
+// lane exchanges inside the wave (DPP moves and row swaps, no LDS), and only
+// the rest goes through LDS (own keys out in 16-byte units, unit u of thread t
+// at u * T + t so that a wave's accesses are consecutive; the partner's in;
+// two barriers).  1024 keys: 3 barrier stages of 55.  Bound by VALU issue and
+// the lane exchanges' latency; with the general shuffle (an LDS access and its
+// address each) and the direction decided per stage, the 1024-key sort of the
+// first-pass sample took 10.0 us, now 2.7 us.
 template <class K, int E>
 __device__ void bitonic_sort_shfl(K* s, uint32_t M) {
-  const uint32_t t = threadIdx.x, base = t * E;
-  const bool own = base < M;  // uniform per wave: M / E is a multiple of 64
+  constexpr int KU = E * sizeof(K) < 16 ? E : (int)(16 / sizeof(K));  // keys per unit
+  constexpr int NU = E / KU;
+  struct alignas(KU * sizeof(K)) Unit { K k[KU]; };
+  Unit* su = reinterpret_cast<Unit*>(s);
+  const uint32_t t = threadIdx.x, T = M / E;
+  const bool own = t < T;  // uniform per wave: T is a multiple of 64
   K r[E];
   if (own) {
 #pragma unroll
-    for (int i = 0; i < E; ++i) r[i] = s[base + i];
-    for (uint32_t size = 2; size <= (uint32_t)E; size <<= 1) bitonic_reg_merge<K, E>(r, base, size, size >> 1);
+    for (int u = 0; u < NU; ++u) {
+      const Unit v = su[t * NU + u];
+#pragma unroll
+      for (int q = 0; q < KU; ++q) r[u * KU + q] = v.k[q];
+    }
+    sort_regs<K, E>(r);
+    sort_lanes<K, E>(r);
   }
-  for (uint32_t size = 2 * E; size <= M; size <<= 1) {
-    const bool asc = (base & size) == 0;
-    for (uint32_t stride = size >> 1; stride >= (uint32_t)E; stride >>= 1) {
-      const uint32_t j = stride / E;
-      const bool keep_min = ((t & j) == 0) == asc;
-      if (j >= 64) {
-        if (own) {
+  // exchange with thread o through LDS; mirrored: key i with its key E - 1 - i
+  auto exchange = [&](uint32_t o, bool mirror, bool keep_min) {
+    const K bound = pair_bound<K>(keep_min);
+    __syncthreads();  // the previous exchange (or the load) is read
+    if (own) {
 #pragma unroll
-          for (int i = 0; i < E; ++i) s[base + i] = r[i];
-        }
-        __syncthreads();
-        K p[E];
-        if (own) {
+      for (int u = 0; u < NU; ++u) {
+        Unit v;
 #pragma unroll
-          for (int i = 0; i < E; ++i) p[i] = s[(t ^ j) * E + i];
-        }
-        __syncthreads();  // every partner read done before the next stage writes
-        if (own) {
-#pragma unroll
-          for (int i = 0; i < E; ++i) r[i] = keep_min ? (p[i] < r[i] ? p[i] : r[i]) : (p[i] > r[i] ? p[i] : r[i]);
-        }
-      } else if (own) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-          const K o = shfl_xor_key<K>(r[i], (int)j);
-          r[i] = keep_min ? (o < r[i] ? o : r[i]) : (o > r[i] ? o : r[i]);
-        }
+        for (int q = 0; q < KU; ++q) v.k[q] = r[u * KU + q];
+        su[u * T + t] = v;
       }
     }
-    if (own) bitonic_reg_merge<K, E>(r, base, size, E / 2);
+    __syncthreads();
+    if (own) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const Unit v = su[(mirror ? NU - 1 - u : u) * T + o];
+#pragma unroll
+        for (int q = 0; q < KU; ++q)
+          r[u * KU + q] = pair_keep<K>(r[u * KU + q], mirror ? v.k[KU - 1 - q] : v.k[q], bound);
+      }
+    }
+  };
+  for (uint32_t lanes = 128; lanes <= T; lanes <<= 1) {  // threads of a run after this merge
+    exchange(t ^ (lanes - 1), true, (t & (lanes >> 1)) == 0);
+    for (uint32_t j = lanes >> 2; j >= 64; j >>= 1) exchange(t ^ j, false, (t & j) == 0);
+    if (own) merge_lanes<K, E, 32>(r);
   }
+  __syncthreads();
   if (own) {
 #pragma unroll
-    for (int i = 0; i < E; ++i) s[base + i] = r[i];
+    for (int u = 0; u < NU; ++u) {
+      Unit v;
+#pragma unroll
+      for (int q = 0; q < KU; ++q) v.k[q] = r[u * KU + q];
+      su[t * NU + u] = v;
+    }
   }
   __syncthreads();
 }

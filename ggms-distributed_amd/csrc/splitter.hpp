@@ -333,9 +333,9 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
         if ((K)(q[j + 1] - q[i]) >= 2) { cnt += 1; nint += 1; }
       } else { cnt += 1; nint += 1; }
     }
-    uint32_t total, ints;
-    uint32_t at = pre + block_excl_scan_u32(cnt, scan_tmp, &total);
-    (void)block_excl_scan_u32(nint, scan_tmp, &ints);
+    uint32_t both;  // at most kPlan0MaxRanges of either: 16 bits each
+    uint32_t at = pre + (block_excl_scan_u32((nint << 16) | cnt, scan_tmp, &both) & 0xFFFFu);
+    const uint32_t total = both & 0xFFFFu, ints = both >> 16;
     const uint32_t share = ints ? (a.B / ints > 0 ? a.B / ints : 1u) : 1u;
     for (uint32_t i = i0; i < i1; ++i) {
       if (i > 0 && q[i] == q[i - 1]) continue;
