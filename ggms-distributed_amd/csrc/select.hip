@@ -140,8 +140,8 @@ static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_o
   uint32_t pieces = (c.mode == kModeLinear || c.mode == kModeStrided) ? std::max<uint32_t>(1, c.P - 1) : c.P;
   c.E = std::max<uint32_t>(1, c.B / pieces / 8);
   uint32_t Q = (c.mode == kModeLinear || c.mode == kModeStrided) ? c.P : c.P + 1;
-  c.R0_bound = 2 * Q + 6;
-  c.B0_bound = c.B + 2 * c.E + 4 + Q;
+  c.R0_bound = 2 * Q + 10;                // up to three edge ranges a side, and two for NaNs
+  c.B0_bound = c.B + 2 * c.E + 8 + Q;
   c.NT = o.block_threads ? o.block_threads : 1024;
   if (c.NT % 64 || c.NT < 64 || c.NT > 1024) c.NT = 1024;
   uint32_t bpc = o.blocks_per_cu ? o.blocks_per_cu : (big_seg ? 1u : 2u);

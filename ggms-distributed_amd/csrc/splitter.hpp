@@ -14,8 +14,8 @@
 // exact results; only the amount of work changes):
 //   * pivots and slopes live in key space and the slope is fixed point;
 //   * the sample extremes replace the global min/max (no extra full pass):
-//     keys below the sample minimum / above the sample maximum fall into two
-//     edge ranges, and keys outside [key(-inf), key(+inf)] (NaNs) into two
+//     keys below the sample minimum / above the sample maximum fall into
+//     edge ranges (up to three a side, see edge_cut), and keys outside [key(-inf), key(+inf)] (NaNs) into two
 //     one-bucket ranges that the plan kernel reports;
 //   * a pivot value that repeats (a value holding >= 1/16 of the sample)
 //     becomes its own one-key range, so a dominant duplicate is resolved
@@ -31,7 +31,8 @@ constexpr int kMlpIn = 65, kMlpHidden = 32, kMlpWin = 64;
 constexpr int kMlpParams = kMlpHidden * kMlpIn + kMlpHidden + kMlpHidden + 1;
 
 // LDS of k_plan0: sorted sample, pivots (<= 2048), range starts, requested and
-// final bucket counts (at most 2 * 1025 + 6 ranges).
+// final bucket counts (at most one or two ranges per run of
+// equal pivots, six edge ranges and two for NaNs).
 constexpr uint32_t kPlan0MaxRanges = 2064;
 // learned pivots are evaluated in chunks of this many (features of a chunk in LDS)
 constexpr uint32_t kMlpChunk = 128;
@@ -131,6 +132,30 @@ __device__ void learned_pivots(const K* s, uint32_t S, uint32_t Pl, const float*
     }
     __syncthreads();
   }
+}
+
+// The keys beyond a sample extreme in up to three ranges: `near` next to it,
+// `mid` behind that, `far` the rest.  They number about n / S and crowd at the
+// extreme, so a single range over all of them puts nearly all into its first
+// bucket: the 1024 largest of 10^7 lognormal values lay in one bucket of ~11000
+// keys, and one value of small integers just above the sample's largest shared
+// its bucket with thousands of unused keys and was bucketed twice more (2^26
+// values in [0, 1024): 290 us a call instead of 123).  `near` spans what the
+// outermost 1/64 of the sample spans, at least one key a bucket, and has half
+// the E buckets; `mid` spans eight times that.
+template <class K> struct EdgeCut {
+  K near, mid, far;  // keys of each
+  __device__ __forceinline__ uint32_t ranges() const { return (near > 0) + (mid > 0) + (far > 0); }
+};
+template <class K> __device__ __forceinline__ EdgeCut<K> edge_cut(K keys, K span, uint32_t E) {
+  EdgeCut<K> c;
+  const K one_each = E / 2 > 0 ? (K)(E / 2) : (K)1;
+  const K want = span > one_each ? span : one_each;
+  c.near = want < keys ? want : keys;
+  const K rest = keys - c.near;
+  c.mid = (rest >> 3) < c.near ? rest : (K)(c.near << 3);
+  c.far = rest - c.mid;
+  return c;
 }
 
 template <class T>
@@ -318,7 +343,10 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
   __syncthreads();
   {
     enum : uint32_t { kSingle = 0, kEdge = 1, kInterior = 2, kNan = 3 };
-    const uint32_t pre = (KT::kFloat ? 1u : 0u) + (q[0] > lowest ? 1u : 0u);
+    const uint32_t tail = (S - 1) / 64 > 0 ? (S - 1) / 64 : (S > 1 ? 1u : 0u);
+    const EdgeCut<K> bot = edge_cut<K>((K)(q[0] - lowest), (K)(s[tail] - s[0]), a.E);
+    const EdgeCut<K> top = edge_cut<K>((K)(highest - q[Q - 1]), (K)(s[S - 1] - s[S - 1 - tail]), a.E);
+    const uint32_t pre = (KT::kFloat ? 1u : 0u) + bot.ranges();
     const uint32_t per_q = (Q + blockDim.x - 1) / blockDim.x;
     const uint32_t i0 = threadIdx.x * per_q, i1 = i0 + per_q < Q ? i0 + per_q : Q;
     uint32_t cnt = 0, nint = 0;
@@ -354,9 +382,15 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
     if (threadIdx.x == 0) {
       uint32_t r = 0;
       if (KT::kFloat) { rlo[r] = (K)0; rreq[r++] = 1; }
-      if (q[0] > lowest) { rlo[r] = lowest; rreq[r++] = a.E; }
+      const uint32_t e2 = a.E / 2 > 0 ? a.E / 2 : 1u, e4 = a.E / 4 > 0 ? a.E / 4 : 1u;
+      if (bot.far) { rlo[r] = lowest; rreq[r++] = e4; }
+      if (bot.mid) { rlo[r] = (K)(lowest + bot.far); rreq[r++] = e4; }
+      if (bot.near) { rlo[r] = (K)(lowest + bot.far + bot.mid); rreq[r++] = e2; }
       r = pre + total;
-      if (q[Q - 1] < highest) { rlo[r] = (K)(q[Q - 1] + 1); rreq[r++] = a.E; }
+      const K beyond = (K)(q[Q - 1] + 1);
+      if (top.near) { rlo[r] = beyond; rreq[r++] = e2; }
+      if (top.mid) { rlo[r] = (K)(beyond + top.near); rreq[r++] = e4; }
+      if (top.far) { rlo[r] = (K)(beyond + top.near + top.mid); rreq[r++] = e4; }
       if (KT::kFloat) { rlo[r] = (K)(highest + 1); rreq[r++] = 1; }
       bcast_R = r;
     }
