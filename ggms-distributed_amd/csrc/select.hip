@@ -540,8 +540,10 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
   const uint32_t fin_grid = std::max<uint32_t>(1, std::min<uint32_t>(4 * (uint32_t)cus, 65535));
   const size_t fin_lds = (size_t)(c.fin_cap / 2) * sizeof(K);
   set_lds_attr((const void*)k_finish<T>, fin_lds);
+  const size_t wide_lds = (size_t)finish_sort_cap<K>() * sizeof(K);
+  set_lds_attr((const void*)k_finish_wide<T>, wide_lds);
   if (n <= c.fin_cap) {
-    const bool wide = finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
+    const bool wide = nk > kSelectMaxKs || finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
     prof.begin(GGMS_KERNEL_OTHER, -1);
     k_tiny_setup<T><<<1, 1024, 0, st>>>(d_vec, n, nk, bufA, k_rank, k_state, (uint32_t*)P(bSmallStart),
                                         (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
@@ -549,13 +551,14 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
     prof.end();
     HIP_TRY(hipGetLastError());
     prof.begin(GGMS_KERNEL_FINISH, 0);
-    k_finish<T><<<1, 1024, fin_lds, st>>>(
-        bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-        (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, flags);
     if (wide)
-      k_finish_wide<T><<<1, 1024, 0, st>>>(bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen),
-                                           (K*)P(bSmallKlo), (K*)P(bSmallKhi), (uint32_t*)P(bSmallKStart), nullptr,
-                                           klist, k_rank, k_state, d_out, c.fin_cap);
+      k_finish_wide<T><<<1, 1024, wide_lds, st>>>(
+          bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
+          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap);
+    else
+      k_finish<T><<<1, 1024, fin_lds, st>>>(
+          bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
+          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, flags);
     prof.end();
     HIP_TRY(hipGetLastError());
     return GGMS_OK;
@@ -674,7 +677,7 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
       k_finish<T><<<fin_grid, 1024, fin_lds, st>>>(dst, cp, pl.small_start, pl.small_len, pl.small_klo,
                                                     pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
                                                     k_state, d_out, c.fin_cap, flags);
-      k_finish_wide<T><<<(uint32_t)cus, 1024, 0, st>>>(dst, src, cp, pl.small_start, pl.small_len, pl.small_klo,
+      k_finish_wide<T><<<(uint32_t)cus, 1024, wide_lds, st>>>(dst, src, cp, pl.small_start, pl.small_len, pl.small_klo,
                                                         pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
                                                         k_state, d_out, c.fin_cap);
       prof.end();
@@ -867,9 +870,11 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
   const uint32_t fin_grid = std::max<uint32_t>(1, std::min<uint32_t>(4 * (uint32_t)ctx->cus, 65535));
   const size_t fin_lds = (size_t)(c.fin_cap / 2) * sizeof(K);  // two workgroups per CU
   set_lds_attr((const void*)k_finish<T>, fin_lds);
+  const size_t wide_lds = (size_t)finish_sort_cap<K>() * sizeof(K);
+  set_lds_attr((const void*)k_finish_wide<T>, wide_lds);
 
   if (n <= c.fin_cap) {
-    const bool wide = finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
+    const bool wide = nk > kSelectMaxKs || finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
     prof.begin(GGMS_KERNEL_OTHER, -1);
     k_tiny_setup<T><<<1, 1024, 0, st>>>(d_vec, n, nk, bufA, k_rank, k_state, (uint32_t*)P(bSmallStart),
                                         (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
@@ -877,13 +882,14 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
     prof.end();
     HIP_TRY(hipGetLastError());
     prof.begin(GGMS_KERNEL_FINISH, 0);
-    k_finish<T><<<1, 1024, fin_lds, st>>>(
-        bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-        (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, dflag);
     if (wide)
-      k_finish_wide<T><<<1, 1024, 0, st>>>(bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen),
-                                           (K*)P(bSmallKlo), (K*)P(bSmallKhi), (uint32_t*)P(bSmallKStart), nullptr,
-                                           klist, k_rank, k_state, d_out, c.fin_cap);
+      k_finish_wide<T><<<1, 1024, wide_lds, st>>>(
+          bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
+          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap);
+    else
+      k_finish<T><<<1, 1024, fin_lds, st>>>(
+          bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
+          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, dflag);
     prof.end();
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
@@ -1061,7 +1067,7 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
               klist, k_rank, k_state, d_out, half ? c.fin_cap / 2 : c.fin_cap, dflag);
         }
         if (h.U_wide > 0)
-          k_finish_wide<T><<<std::min<uint32_t>(h.U_wide, (uint32_t)ctx->cus), 1024, 0, st>>>(
+          k_finish_wide<T><<<std::min<uint32_t>(h.U_wide, (uint32_t)ctx->cus), 1024, wide_lds, st>>>(
               dst, src, cp, pl.small_start, pl.small_len, pl.small_klo, pl.small_khi, pl.small_kstart, pl.small_order,
               klist, k_rank, k_state, d_out, c.fin_cap);
         prof.end();

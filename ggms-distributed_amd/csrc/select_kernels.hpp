@@ -416,12 +416,12 @@ __device__ __forceinline__ K lane_xor_key(K v) {
 // median of the two and the bound, one v_med3_u32 for 32-bit keys.
 template <class K> __device__ __forceinline__ K pair_bound(bool keep_min) { return keep_min ? (K)0 : (K)~(K)0; }
 template <class K> __device__ __forceinline__ K pair_keep(K a, K b, K bound) {
-  const K lo = a < b ? a : b, hi = a < b ? b : a;
   if constexpr (sizeof(K) == 4) {
+    const K lo = a < b ? a : b, hi = a < b ? b : a;
     const K m = hi < bound ? hi : bound;
     return lo < m ? m : lo;
   } else {
-    return bound ? hi : lo;
+    return (a < b) != (bound != 0) ? a : b;
   }
 }
 // Registers [0, E): the compare-exchanges at distances from, from / 2, .., 1,
@@ -572,10 +572,12 @@ template <class K, bool SW = false, bool SHFL = true>
 __device__ void bitonic_sort_lds(K* s, uint32_t M) {
   const uint32_t e = M / blockDim.x;
   if (M == e * blockDim.x &&
-      (e == 4 || e == 8 || (e == 16 && sizeof(K) <= 4) || (e == 32 && sizeof(K) == 2))) {
+      (e == 4 || e == 8 || (e == 16 && (sizeof(K) <= 4 || SHFL)) ||
+       (e == 32 && (sizeof(K) == 2 || (sizeof(K) == 4 && SHFL))))) {
     if (SHFL && e == 4) bitonic_sort_shfl<K, 4>(s, M);
     else if (SHFL && e == 8) bitonic_sort_shfl<K, 8>(s, M);
     else if (SHFL && e == 16) bitonic_sort_shfl<K, 16>(s, M);
+    else if (SHFL && e == 32 && sizeof(K) == 4) bitonic_sort_shfl<K, 32>(s, M);
     else if (e == 4) bitonic_sort_lds_reg<K, 4, SW>(s, M);
     else if (e == 8) bitonic_sort_lds_reg<K, 8, SW>(s, M);
     else if (e == 16) bitonic_sort_lds_reg<K, 16, SW>(s, M);
@@ -600,6 +602,10 @@ __device__ void bitonic_sort_lds(K* s, uint32_t M) {
 template <class K> struct HalfKey;
 template <> struct HalfKey<uint32_t> { using T = uint16_t; };
 template <> struct HalfKey<uint64_t> { using T = uint32_t; };
+
+// ks of a segment that one radix select answers together; a segment with more
+// is sorted.
+constexpr uint32_t kSelectMaxKs = 8;
 
 // The finish holds a segment in fin_cap / 2 full-width keys of LDS (two
 // workgroups per CU): as keys when it has at most fin_cap / 2 of them, or as
@@ -655,6 +661,7 @@ __host__ __device__ __forceinline__ uint32_t order_bin_info(uint32_t len, K klo,
   return base | wave;
 }
 __host__ __device__ __forceinline__ uint32_t order_bin_of(uint32_t info, uint32_t nks, bool waves) {
+  if (nks > kSelectMaxKs) return 0;
   const bool wave = ((info & 0x100u) && nks <= kFinishWaveKs) || ((info & 0x200u) && nks == 1);
   return (waves && wave) ? 1u : (info & 0xFFu);
 }
@@ -2789,7 +2796,6 @@ __global__ void __launch_bounds__(1024) k_compactS(const K* __restrict__ buf, co
 // from its prefix's histogram.  A segment holding many ks is sorted instead
 // (bitonic network in LDS) and read at every rank.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kSelectMaxKs = 8;
 
 // Radix select of one rank (the batched kernel's finish): same digits, one
 // 256-bin histogram per round.
@@ -3050,18 +3056,15 @@ __device__ __forceinline__ void load_segment(const K* __restrict__ buf, uint32_t
   for (uint32_t i = threadIdx.x + kSegLoadVecs * blockDim.x; i < nv; i += blockDim.x) put(i, src[i]);
 }
 
-// Answers the ks [q0, q1) of one segment held in LDS as type C, C value = key - base.
-// s is writable LDS, except for the global-memory case, which passes at most
-// kSelectMaxKs ks and so never reaches the sort.  counted: see
-// radix_select_multi (at most kSelectMaxKs ks).
+// Answers the q <= kSelectMaxKs ks of one segment held in LDS (or global
+// memory) as type C, C value = key - base; thread j < q holds k j's index and
+// rank.  counted: see radix_select_multi.
 template <class T, class C>
 __device__ __forceinline__ void finish_segment(const C* __restrict__ s, uint32_t len, C clo, C chi,
-                                               typename KeyTraits<T>::K base, uint32_t q0, uint32_t q1,
-                                               uint32_t kk, uint32_t kr, const uint32_t* __restrict__ klist,
-                                               uint32_t* __restrict__ k_rank, uint32_t* __restrict__ k_state,
-                                               T* __restrict__ out, SelectLds& L, bool counted = false) {
+                                               typename KeyTraits<T>::K base, uint32_t q, uint32_t kk, uint32_t kr,
+                                               uint32_t* __restrict__ k_state, T* __restrict__ out, SelectLds& L,
+                                               bool counted = false) {
   using K = typename KeyTraits<T>::K;
-  const uint32_t q = q1 - q0;
   if (q == 1) {
     if (threadIdx.x == 0) {
       L.kid[0] = kk;
@@ -3073,7 +3076,7 @@ __device__ __forceinline__ void finish_segment(const C* __restrict__ s, uint32_t
       out[kk] = KeyTraits<T>::dec((K)(base + (K)(C)L.pre[0]));
       k_state[kk] = kDone;
     }
-  } else if (q <= kSelectMaxKs) {
+  } else {
     if (threadIdx.x < q) {
       L.kid[threadIdx.x] = kk;
       L.rank[threadIdx.x] = kr;
@@ -3096,17 +3099,6 @@ __device__ __forceinline__ void finish_segment(const C* __restrict__ s, uint32_t
     if (threadIdx.x < q) {
       const uint32_t k = L.kid[threadIdx.x];
       out[k] = KeyTraits<T>::dec((K)(base + (K)(C)L.pre[threadIdx.x]));
-      k_state[k] = kDone;
-    }
-  } else {
-    C* w = const_cast<C*>(s);
-    const uint32_t M = pow2ceil_u32(len);
-    for (uint32_t i = len + threadIdx.x; i < M; i += blockDim.x) w[i] = (C)~(C)0;
-    __syncthreads();
-    bitonic_sort_lds<C, false, false>(w, M);  // within the 64-VGPR budget: plain LDS stages
-    for (uint32_t qq = q0 + threadIdx.x; qq < q1; qq += blockDim.x) {
-      const uint32_t k = klist[qq];
-      out[k] = KeyTraits<T>::dec((K)(base + (K)s[k_rank[k] - 1]));
       k_state[k] = kDone;
     }
   }
@@ -3184,29 +3176,28 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8)
     }
     const K klo = g.klo, khi = g.khi;
     const uint32_t q0 = g.q0, q1 = g.q1;
-    if (!finish_fits_half<K>(len, klo, khi, fin_cap)) continue;  // k_finish_wide's
+    if (!finish_fits_half<K>(len, klo, khi, fin_cap) || q1 - q0 > kSelectMaxKs) continue;  // k_finish_wide's
     // the ks and their ranks are fetched while the segment loads
     uint32_t kk = 0, kr = 0;
-    if (threadIdx.x < q1 - q0 && q1 - q0 <= kSelectMaxKs) {
+    if (threadIdx.x < q1 - q0) {
       kk = klist[q0 + threadIdx.x];
       kr = k_rank[kk];
     }
-    // The segment is loaded into LDS as C values (key - base).  With at most
-    // kSelectMaxKs ks the load also counts the radix select's first digit,
-    // and stores the keys only when later digits need them.
+    // The segment is loaded into LDS as C values (key - base).  The load also
+    // counts the radix select's first digit, and stores the keys only when
+    // later digits need them.
     auto run = [&](auto* sv, auto clo, auto chi, K base) {
       using C = typename std::remove_pointer<decltype(sv)>::type;
-      const bool sel = q1 - q0 <= kSelectMaxKs;
       uint32_t sh1, w1;
       select_first_digit(bitlen64((uint64_t)(clo ^ chi)), sh1, w1);
-      const bool keep = !sel || sh1 > 0;
+      const bool keep = sh1 > 0;
       load_segment<K>(buf, st, len, [&](uint32_t i, K key, bool in) {
         const C c = (C)(key - base);
         if (in && keep) sv[i] = c;
-        if (sel) select_count_first<C>(L.hist, c, sh1, w1, in);
+        select_count_first<C>(L.hist, c, sh1, w1, in);
       });
-      finish_segment<T, C>(sv, len, clo, chi, base, q0, q1, kk, kr, klist, k_rank, k_state, out, L, sel);
-      if (sel) select_zero_first(L);  // for the next segment (the barrier below orders it)
+      finish_segment<T, C>(sv, len, clo, chi, base, q1 - q0, kk, kr, k_state, out, L, true);
+      select_zero_first(L);  // for the next segment (the barrier below orders it)
     };
     if (len > fin_cap / 2) run(reinterpret_cast<H*>(smem), (H)0, (H)(khi - klo), klo);  // narrow interval
     else run(reinterpret_cast<K*>(smem), klo, khi, (K)0);
@@ -3307,15 +3298,20 @@ __device__ const K* wg_radix_sort_global(K* __restrict__ a, K* __restrict__ tmp,
   return src;
 }
 
-// Small segments too wide for half-width offsets and too large for full keys
-// in the finish kernel's LDS (rare: a few per call at most), and segments
-// larger than the finish capacity (the one-pass bucketMultiselect, or a pass
-// cap that forced finishing), from global memory: up to kSelectMaxKs ks by
-// radix select (one sweep per digit for all of them); more ks (a k-dense
-// segment, e.g. the top segment of a top-k select) by a stable radix sort of
-// the segment through the same positions of the spare buffer `tmp`, read at
-// every rank.  They are the last U_wide entries of the finish order; one
-// workgroup per segment.
+// The segments k_finish leaves: more ks than one radix select answers
+// (k-dense: the top segment of a top-k select, or ranks clustered in a window),
+// or too wide for half-width offsets and too large for full keys in its LDS
+// (rare), or larger than the finish capacity (the one-pass bucketMultiselect,
+// or a pass cap that forced finishing).  A k-dense segment of up to
+// finish_sort_cap keys is sorted in LDS in registers (bitonic_sort_shfl; one
+// workgroup a CU for its 128 KB and its registers) and read at every rank: in
+// k_finish, held to 64 VGPRs and LDS stages, 11000 keys with 1000 ks took
+// 155 us, here 43 (32768 keys 256 -> 84).  A longer one takes a stable radix sort through the same positions
+// of the spare buffer `tmp`.  Few ks are radix-selected (one sweep per digit for
+// all of them, up to kSelectMaxKs a time) from the same LDS, or from global
+// memory above its size.  They are the last U_wide entries of the finish
+// order; one workgroup per segment.
+template <class K> __host__ __device__ constexpr uint32_t finish_sort_cap() { return sizeof(K) == 4 ? 32768u : 16384u; }
 template <class T>
 __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* __restrict__ buf,
                                                       typename KeyTraits<T>::K* __restrict__ tmp,
@@ -3330,6 +3326,7 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
                                                       uint32_t* __restrict__ k_state, T* __restrict__ out,
                                                       uint32_t fin_cap) {
   using K = typename KeyTraits<T>::K;
+  extern __shared__ __align__(16) unsigned char smem[];  // finish_sort_cap keys
   __shared__ SelectLds L;
   __shared__ RadixSortLds RL;
   const uint32_t U_small = ctl->U_small, U_wide = ctl->U_wide;
@@ -3337,15 +3334,51 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
     const uint32_t j = small_order ? small_order[jj] : jj;
     const uint32_t st = small_start[j], len = small_len[j];
     const K klo = small_klo[j], khi = small_khi[j];
-    if (!finish_wide_segment<K>(len, klo, khi, fin_cap)) continue;  // k_finish's
     const uint32_t q0 = small_kstart[j], q1 = small_kstart[j + 1];
-    if (q1 - q0 > kSelectMaxKs && tmp) {
+    const bool dense = q1 - q0 > kSelectMaxKs;
+    if (!dense && !finish_wide_segment<K>(len, klo, khi, fin_cap)) continue;  // k_finish's
+    if (dense && len <= finish_sort_cap<K>()) {
+      K* s = reinterpret_cast<K*>(smem);
+      load_segment<K>(buf, st, len, [&](uint32_t i, K key, bool in) {
+        if (in) s[i] = key;
+      });
+      const uint32_t M = pow2ceil_u32(len);
+      for (uint32_t i = len + threadIdx.x; i < M; i += blockDim.x) s[i] = KeyMax<K>::v;
+      __syncthreads();
+      bitonic_sort_lds<K>(s, M);
+      for (uint32_t qq = q0 + threadIdx.x; qq < q1; qq += blockDim.x) {
+        const uint32_t k = klist[qq];
+        out[k] = KeyTraits<T>::dec(s[k_rank[k] - 1]);
+        k_state[k] = kDone;
+      }
+      __syncthreads();
+      continue;
+    }
+    if (dense && tmp) {
       const K* sorted = wg_radix_sort_global<K>(buf + st, tmp + st, len, bitlen64((uint64_t)(klo ^ khi)), RL);
       for (uint32_t qq = q0 + threadIdx.x; qq < q1; qq += blockDim.x) {
         const uint32_t k = klist[qq];
         out[k] = KeyTraits<T>::dec(sorted[k_rank[k] - 1]);
         k_state[k] = kDone;
       }
+      __syncthreads();
+      continue;
+    }
+    if (len <= finish_sort_cap<K>()) {  // few ks, one load into LDS as in k_finish
+      K* s = reinterpret_cast<K*>(smem);
+      uint32_t kk = 0, kr = 0, sh1, w1;
+      if (threadIdx.x < q1 - q0) {
+        kk = klist[q0 + threadIdx.x];
+        kr = k_rank[kk];
+      }
+      select_zero_first(L);
+      __syncthreads();
+      select_first_digit(bitlen64((uint64_t)(klo ^ khi)), sh1, w1);
+      load_segment<K>(buf, st, len, [&](uint32_t i, K key, bool in) {
+        if (in) s[i] = key;
+        select_count_first<K>(L.hist, key, sh1, w1, in);
+      });
+      finish_segment<T, K>(s, len, klo, khi, (K)0, q1 - q0, kk, kr, k_state, out, L, true);
       __syncthreads();
       continue;
     }
@@ -3356,7 +3389,7 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
         kk = klist[c0 + threadIdx.x];
         kr = k_rank[kk];
       }
-      finish_segment<T, K>(buf + st, len, klo, khi, (K)0, c0, c1, kk, kr, klist, k_rank, k_state, out, L);
+      finish_segment<T, K>(buf + st, len, klo, khi, (K)0, c1 - c0, kk, kr, k_state, out, L);
       __syncthreads();
     }
   }
