@@ -489,6 +489,27 @@ static size_t pass1_lds_fixed(const Config& c, size_t own) {
   return std::max<size_t>(base, kPass1ParamsLds);
 }
 
+// A call of at most the finish capacity: one launch.  flags: as launch_fixed's.
+template <class T>
+static ggms_status launch_tiny(const T* d_vec, uint32_t n, const uint32_t* d_ks, uint32_t nk, T* d_out,
+                               uint32_t* k_state, uint32_t* flags, hipStream_t st, Prof& prof) {
+  const size_t lds = (size_t)tiny_keys(n) * sizeof(T);
+  set_lds_attr((const void*)k_tiny<T>, lds);
+  prof.begin(GGMS_KERNEL_FINISH, 0);
+  k_tiny<T><<<1, 1024, lds, st>>>(d_vec, n, d_ks, nk, d_out, k_state, flags);
+  prof.end();
+  HIP_TRY(hipGetLastError());
+  return GGMS_OK;
+}
+
+template <class T>
+static ggms_status launch_segmented_first_pass(const Config& c, const Layout& L, char* W, const T* d_vec,
+                                               uint32_t n, uint32_t G0, PassCtl* cp, PlanArgs<typename KeyTraits<T>::K>& pl,
+                                               typename KeyTraits<T>::K* scratch, typename KeyTraits<T>::K* dst,
+                                               hipStream_t st, Prof& prof);
+template <class K>
+static void plan_groups(PlanArgs<K>& pl, const Layout& L, char* W, bool on);
+
 // The whole call enqueued on `st` with no host reads between kernels (a
 // device-driven schedule): every pass's kernels are launched with shapes and
 // LDS sized for the largest pass the call can produce; a kernel whose pass
@@ -525,11 +546,12 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
   c0.nan_lo_bucket = kNone32;
   c0.nan_hi_bucket = kNone32;
   c0.hot_bucket = kNone32;
+  if (n <= c.fin_cap) return launch_tiny<T>(d_vec, n, d_ks, nk, d_out, k_state, flags, st, prof);
   // the status words start clear (a fill kernel: capturable, unlike a memset)
   k_fill_u32<<<1, 64, 0, st>>>(flags, 3, 0u);
   HIP_TRY(hipGetLastError());
   const uint32_t ctl_words = (uint32_t)((c.max_passes + 2) * ctlb / 4);
-  const bool setup_in_plan0 = n > c.fin_cap && nk <= kSetupInPlan0MaxKs;
+  const bool setup_in_plan0 = nk <= kSetupInPlan0MaxKs;
   if (!setup_in_plan0) {
     prof.begin(GGMS_KERNEL_OTHER, -1);
     const uint32_t threads = std::max(ctl_words, nk);
@@ -542,27 +564,6 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
   set_lds_attr((const void*)k_finish<T>, fin_lds);
   const size_t wide_lds = (size_t)finish_sort_cap<K>() * sizeof(K);
   set_lds_attr((const void*)k_finish_wide<T>, wide_lds);
-  if (n <= c.fin_cap) {
-    const bool wide = nk > kSelectMaxKs || finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
-    prof.begin(GGMS_KERNEL_OTHER, -1);
-    k_tiny_setup<T><<<1, 1024, 0, st>>>(d_vec, n, nk, bufA, k_rank, k_state, (uint32_t*)P(bSmallStart),
-                                        (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-                                        (uint32_t*)P(bSmallKStart), klist, ctl, wide ? 1u : 0u);
-    prof.end();
-    HIP_TRY(hipGetLastError());
-    prof.begin(GGMS_KERNEL_FINISH, 0);
-    if (wide)
-      k_finish_wide<T><<<1, 1024, wide_lds, st>>>(
-          bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap);
-    else
-      k_finish<T><<<1, 1024, fin_lds, st>>>(
-          bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, flags);
-    prof.end();
-    HIP_TRY(hipGetLastError());
-    return GGMS_OK;
-  }
   const Plan0Args pa = plan0_args<T>(c, device, nk, ctl_words, setup_in_plan0, d_ks, k_rank, k_state, flags + 1, c0);
   const size_t lds_p0 = plan0_lds_bytes<K>(pow2ceil_host(c.S));
   LDS_CHECK(lds_p0);
@@ -845,6 +846,17 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
     return fixed_status((const uint32_t*)hflag);
   }
 
+  if (n <= c.fin_cap) {
+    s = launch_tiny<T>(d_vec, n, d_ks, nk, d_out, k_state, dflag, st, prof);
+    if (s) return s;
+    HIP_TRY(hipStreamSynchronize(st));
+    if (*hbad) return GGMS_EINVAL;
+    if (!out_on_device) memcpy(out, hout, (size_t)nk * sizeof(T));
+    stt.finished_segments = 1;
+    prof.collect(stt);
+    return GGMS_OK;
+  }
+
   // control block 0
   PassCtl c0{};
   c0.n = n;
@@ -858,7 +870,7 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
   // setup (control blocks, ks -> ranks): its own kernel, or folded into the
   // first-pass planning kernel when the ks are few enough for one workgroup
   const uint32_t ctl_words = (uint32_t)((c.max_passes + 2) * ctlb / 4);
-  const bool setup_in_plan0 = n > c.fin_cap && nk <= kSetupInPlan0MaxKs;
+  const bool setup_in_plan0 = nk <= kSetupInPlan0MaxKs;
   if (!setup_in_plan0) {
     prof.begin(GGMS_KERNEL_OTHER, -1);
     const uint32_t threads = std::max(ctl_words, nk);
@@ -873,233 +885,207 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
   const size_t wide_lds = (size_t)finish_sort_cap<K>() * sizeof(K);
   set_lds_attr((const void*)k_finish_wide<T>, wide_lds);
 
-  if (n <= c.fin_cap) {
-    const bool wide = nk > kSelectMaxKs || finish_wide_segment<K>(n, (K)0, KeyMax<K>::v, c.fin_cap);
-    prof.begin(GGMS_KERNEL_OTHER, -1);
-    k_tiny_setup<T><<<1, 1024, 0, st>>>(d_vec, n, nk, bufA, k_rank, k_state, (uint32_t*)P(bSmallStart),
-                                        (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-                                        (uint32_t*)P(bSmallKStart), klist, ctl, wide ? 1u : 0u);
-    prof.end();
-    HIP_TRY(hipGetLastError());
-    prof.begin(GGMS_KERNEL_FINISH, 0);
-    if (wide)
-      k_finish_wide<T><<<1, 1024, wide_lds, st>>>(
-          bufA, bufB, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap);
-    else
-      k_finish<T><<<1, 1024, fin_lds, st>>>(
-          bufA, ctl, (uint32_t*)P(bSmallStart), (uint32_t*)P(bSmallLen), (K*)P(bSmallKlo), (K*)P(bSmallKhi),
-          (uint32_t*)P(bSmallKStart), nullptr, klist, k_rank, k_state, d_out, c.fin_cap, dflag);
-    prof.end();
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(st));
-    if (*hbad) return GGMS_EINVAL;
-    if (*hflag) return GGMS_EDEVICE;
-    stt.passes = 0;
-    stt.finished_segments = 1;
-  } else {
-    // first-pass splitter
-    const Plan0Args pa = plan0_args<T>(c, ctx->device, nk, ctl_words, setup_in_plan0, d_ks, k_rank, k_state, dbad, c0);
-    size_t lds_p0 = plan0_lds_bytes<K>(pow2ceil_host(c.S));
-    LDS_CHECK(lds_p0);
-    set_lds_attr((const void*)k_plan0<T>, lds_p0);
-    prof.begin(GGMS_KERNEL_PLAN0, 0);
-    k_plan0<T><<<1, 1024, lds_p0, st>>>(d_vec, pa, rng_first, (K*)P(bLut), ctl);
-    prof.end();
-    HIP_TRY(hipGetLastError());
+  // first-pass splitter
+  const Plan0Args pa = plan0_args<T>(c, ctx->device, nk, ctl_words, setup_in_plan0, d_ks, k_rank, k_state, dbad, c0);
+  size_t lds_p0 = plan0_lds_bytes<K>(pow2ceil_host(c.S));
+  LDS_CHECK(lds_p0);
+  set_lds_attr((const void*)k_plan0<T>, lds_p0);
+  prof.begin(GGMS_KERNEL_PLAN0, 0);
+  k_plan0<T><<<1, 1024, lds_p0, st>>>(d_vec, pa, rng_first, (K*)P(bLut), ctl);
+  prof.end();
+  HIP_TRY(hipGetLastError());
 
-    uint32_t G = G0, B_bound = c.B0_bound, R_bound = c.R0_bound;
-    uint32_t B0 = c.B0_bound, R0 = c.R0_bound, L2 = LutGeom<K>::L2TABLES;  // exact after pass 0
-    uint16_t* slot_tab[2] = {(uint16_t*)P(bSlotOfBucket),
-                             (uint16_t*)P(bSlotOfBucket) + (std::max<size_t>(c.B0_bound, c.B_cap) + 64)};
-    uint32_t U_slot_bound = std::min<uint32_t>(nk, B_bound);
-    for (uint32_t pass = 0;; ++pass) {
-      PassCtl* cp = ctl + pass;
-      PassCtl* cn = ctl + pass + 1;
-      Range<K>* rc = pass == 0 ? rng_first : rng[pass & 1];
-      Range<K>* rn = rng[(pass + 1) & 1];
-      K* src = (pass & 1) ? bufA : bufB;  // input of pass >= 1
-      K* dst = (pass & 1) ? bufB : bufA;  // output of this pass's compaction
-      // tile -> first range table: read by this pass's streaming kernels, written
-      // by this pass's plan for the next pass (so it must not alias)
-      uint32_t* wgf_cur = (uint32_t*)P(bWgFirst) + (size_t)(pass & 1) * c.G_max;
-      uint32_t* wgf_next = (uint32_t*)P(bWgFirst) + (size_t)((pass + 1) & 1) * c.G_max;
-      const uint32_t NT = c.NT;
-      // pass-1 range parameters live in LDS unless that would push either
-      // pass-1 kernel past kPass1ParamsLds (then they are read from global memory)
-      uint32_t p1_lds = 0;
-      if (pass == 1 && !c.seg_first) {
-        size_t cnt = ((size_t)B_bound * 4 + 15) / 16 * 16 + pass1_map_bytes<K>(B0, R0, L2, R_bound);
-        size_t cmp = compact_lds_bytes(B_bound, U_slot_bound + 4) + pass1_map_bytes<K>(B0, R0, L2, R_bound);
-        p1_lds = std::max(cnt, cmp) <= kPass1ParamsLds ? 1u : 0u;
-      }
-      // count
-      if (pass == 0) {
-        size_t lds = count_lds0<T>(c);
-        LDS_CHECK(count_lds0_total<T>(c));
-        // when the tables already allow only one workgroup per CU and a second
-        // histogram still fits, each workgroup counts two consecutive tiles
-        // (one row each) without a barrier between them, so its loads do not
-        // drain and restart at a tile boundary (2^28 fp32: 0.185 -> 0.175 ms)
-        const size_t hist2 = (size_t)c.B0_bound * 4;
-        const uint32_t tpw =
-            (count_lds0_total<T>(c) > kLdsOneWgPerCu && count_lds0_total<T>(c) + hist2 <= kLdsLimit) ? 2u : 1u;
-        if (tpw == 2) lds += hist2;
-        set_lds_attr((const void*)k_count0<T>, lds);
-        prof.begin(GGMS_KERNEL_COUNT0, (int)pass);
-        k_count0<T><<<(G + tpw - 1) / tpw, NT, lds, st>>>(d_vec, rc, (K*)P(bLut), cp, rows, tpw);
-        prof.end();
-      } else if (pass == 1 && !c.seg_first) {
-        size_t lds = ((size_t)B_bound * 4 + 15) / 16 * 16 + pass1_map_bytes<K>(B0, R0, L2, p1_lds ? R_bound : 0);
-        LDS_CHECK(lds);
-        set_lds_attr((const void*)k_count1<K>, lds);
-        prof.begin(GGMS_KERNEL_COUNTS, (int)pass);
-        k_count1<K><<<G, NT, lds, st>>>(src, ctl, (K*)P(bLut), rng_first, (uint64_t*)P(bRank0),
-                                        (MapParam<K>*)P(bParams1), p1_lds ? (uint32_t)lds : 0u, cp, rows);
-        prof.end();
-      } else {
-        size_t lds = (size_t)B_bound * 4;
-        LDS_CHECK(lds);
-        set_lds_attr((const void*)k_countS<K>, lds);
-        prof.begin(GGMS_KERNEL_COUNTS, (int)pass);
-        k_countS<K><<<G, NT, lds, st>>>(src, rc, wgf_cur, cp, rows);
-        prof.end();
-      }
-      HIP_TRY(hipGetLastError());
-      prof.begin(GGMS_KERNEL_COLSUM, (int)pass);
-      k_colsum<<<(B_bound + 63) / 64, 1024, 0, st>>>(rows, cp, totals);
-      prof.end();
-      HIP_TRY(hipGetLastError());
-      // plan
-      PlanArgs<K> pl = plan_args_common<K>(c, L, W, nk, d_out);
-      pl.ranges = rc;
-      pl.ctl = cp;
-      pl.ctl_next = cn;
-      pl.next_ranges = rn;
-      pl.slot_of_bucket = slot_tab[pass & 1];
-      pl.wg_first_next = wgf_next;
-      pl.force_finish = (pass + 1 >= c.max_passes) ? 1u : c.force_finish;
-      pl.finish_cap = (pass == 0 && c.one_pass) ? kOnePassFinishCap * c.fin_cap : c.fin_cap;
-      pl.merge_small = (pass == 0 && !c.seg_first) ? 1u : 0u;
-      pl.next_params = (pass == 0 && !c.seg_first) ? (MapParam<K>*)P(bParams1) : nullptr;
-      pl.rank_words = (pass == 0 && !c.seg_first) ? (uint64_t*)P(bRank0) : nullptr;
-      pl.mirror = dmirror;
-      pl.mirror_seq = dseq;
-      if (++ctx->mirror_seq == 0) ++ctx->mirror_seq;
-      pl.seq = ctx->mirror_seq;
-      pl.nan_out = nullptr;
-      plan_groups<K>(pl, L, W, pass == 0 && c.seg_first);
-      size_t lds_plan = plan_lds_bytes(B_bound, nk);
-      pl.lds_words = (uint32_t)(lds_plan / 4);
-      LDS_CHECK(lds_plan);
-      set_lds_attr((const void*)k_plan<T>, lds_plan);
-      prof.begin(GGMS_KERNEL_PLAN, (int)pass);
-      k_plan<T><<<1, 1024, lds_plan, st>>>(pl);
-      prof.end();
-      HIP_TRY(hipGetLastError());
-      // compaction
-      if (pass == 0 && c.seg_first) {
-        // every k-bucket into its own segment (the finish reads segments)
-        s = launch_segmented_first_pass<T>(c, L, W, d_vec, n, G, cp, pl, src, dst, st, prof);
-        if (s) return s;
-      } else if (pass == 0) {
-        // dynamic part: map parameters then the slot table (cell table is static LDS)
-        size_t lds = (size_t)R_bound * sizeof(MapParam<K>) + (size_t)B_bound * 2;
-        LDS_CHECK(lds + LutGeom<K>::bytes());
-        set_lds_attr((const void*)k_compact0<T>, lds);
-        prof.begin(GGMS_KERNEL_COMPACT0, (int)pass);
-        k_compact0<T><<<G, NT, lds, st>>>(d_vec, rc, (K*)P(bLut), cp, rows, pl.slot_of_bucket, pl.slot_bucket,
-                                          dst);
-        prof.end();
-      } else if (pass == 1 && !c.seg_first) {
-        size_t lds = compact_lds_bytes(B_bound, U_slot_bound + 4) + pass1_map_bytes<K>(B0, R0, L2, p1_lds ? R_bound : 0);
-        // one workgroup per CU: its writes scatter over every k-bucket segment,
-        // and twice the workgroups in flight keep twice the partial HBM lines
-        // open (measured 0.197 ms with two per CU, 0.154 ms with one)
-        lds = std::max<size_t>(lds, kLdsOneWgPerCu);
-        LDS_CHECK(lds);
-        set_lds_attr((const void*)k_compact1<K>, lds);
-        prof.begin(GGMS_KERNEL_COMPACTS, (int)pass);
-        k_compact1<K><<<G, NT, lds, st>>>(src, ctl, (K*)P(bLut), rng_first, (uint64_t*)P(bRank0),
-                                          (MapParam<K>*)P(bParams1), p1_lds ? (uint32_t)lds : 0u, cp, rows,
-                                          pl.slot_of_bucket, pl.slot_dst, pl.slot_bucket, dst);
-        prof.end();
-      } else {
-        size_t lds = compact_lds_bytes(B_bound, U_slot_bound + 4);
-        LDS_CHECK(lds);
-        set_lds_attr((const void*)k_compactS<K>, lds);
-        prof.begin(GGMS_KERNEL_COMPACTS, (int)pass);
-        k_compactS<K><<<G, NT, lds, st>>>(src, rc, wgf_cur, cp, rows, pl.slot_of_bucket,
-                                          pl.slot_dst, pl.slot_bucket, dst);
-        prof.end();
-      }
-      HIP_TRY(hipGetLastError());
-      // the next pass (and this pass's finish) is planned from the control
-      // blocks the plan kernel wrote to host memory, while the compaction
-      // runs.  The host polls the sequence word the plan writes after them:
-      // an event recorded between the plan and the compaction would make the
-      // GPU drain and publish at that point (~6 us idle before each compaction).
-      s = wait_mirror(hseq, pl.seq, st);
-      if (s) return s;
-      const PassCtl h = hmirror[0];
-      const PassCtl hn = hmirror[1];
-      // the iterative first pass hands every k-bucket to pass 1
-      if ((pass > 0 || c.seg_first) && h.U_small > 0) {
-        // every segment within a quarter of the capacity: half-size workgroups
-        // (512 threads, half the LDS) so twice as many run at once
-        const bool half = h.small_max <= c.fin_cap / 4;
-        // many small segments beside a few large ones: the large ones first
-        // (full workgroups), then the small ones in half-size workgroups
-        const uint32_t U_grp = h.U_small - h.U_wave - h.U_wide;
-        const bool split = !half && c.fin_cap / 4 >= kFinishSplitLen &&
-                           U_grp - std::min(h.U_fin_big, U_grp) >= kFinishSplitMinSegs;
-        prof.begin(GGMS_KERNEL_FINISH, (int)pass);
-        if (split) {
-          k_finish<T><<<fin_grid, 1024, fin_lds, st>>>(dst, cp, pl.small_start, pl.small_len, pl.small_klo,
-                                                       pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
-                                                       k_state, d_out, c.fin_cap, dflag, 1u);
-          k_finish<T><<<fin_grid, 512, fin_lds / 2, st>>>(dst, cp, pl.small_start, pl.small_len, pl.small_klo,
-                                                          pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
-                                                          k_state, d_out, c.fin_cap / 2, dflag, 2u);
-        } else {
-          k_finish<T><<<fin_grid, half ? 512 : 1024, half ? fin_lds / 2 : fin_lds, st>>>(
-              dst, cp, pl.small_start, pl.small_len, pl.small_klo, pl.small_khi, pl.small_kstart, pl.small_order,
-              klist, k_rank, k_state, d_out, half ? c.fin_cap / 2 : c.fin_cap, dflag);
-        }
-        if (h.U_wide > 0)
-          k_finish_wide<T><<<std::min<uint32_t>(h.U_wide, (uint32_t)ctx->cus), 1024, wide_lds, st>>>(
-              dst, src, cp, pl.small_start, pl.small_len, pl.small_klo, pl.small_khi, pl.small_kstart, pl.small_order,
-              klist, k_rank, k_state, d_out, c.fin_cap);
-        prof.end();
-        HIP_TRY(hipGetLastError());
-      }
-      if (pass == 0 && (*hbad || h.nan_count)) {
-        HIP_TRY(hipStreamSynchronize(st));
-        return *hbad ? GGMS_EINVAL : GGMS_ENAN;
-      }
-      if (pass == 0) {
-        B0 = h.B;
-        R0 = h.R;
-        L2 = h.l2_used;
-      }
-      if (pass < GGMS_MAX_PASS_STATS) {
-        stt.n_in[pass] = h.n;
-        stt.active[pass] = h.U;
-        stt.n_kept[pass] = (uint64_t)h.N_big + h.N_small;
-        stt.buckets[pass] = h.B;
-      }
-      stt.passes = pass + 1;
-      stt.finished_segments += h.U_small;
-      if (h.N_big == 0 || h.U_big == 0) break;
-      if (pass + 1 >= c.max_passes) {  // cannot happen: the last pass forces finishing
-        HIP_TRY(hipStreamSynchronize(st));
-        return GGMS_EDEVICE;
-      }
-      G = hn.G;
-      B_bound = std::max<uint32_t>(hn.B, 1);
-      R_bound = hn.R;
-      U_slot_bound = std::min<uint32_t>(nk, B_bound);
+  uint32_t G = G0, B_bound = c.B0_bound, R_bound = c.R0_bound;
+  uint32_t B0 = c.B0_bound, R0 = c.R0_bound, L2 = LutGeom<K>::L2TABLES;  // exact after pass 0
+  uint16_t* slot_tab[2] = {(uint16_t*)P(bSlotOfBucket),
+                           (uint16_t*)P(bSlotOfBucket) + (std::max<size_t>(c.B0_bound, c.B_cap) + 64)};
+  uint32_t U_slot_bound = std::min<uint32_t>(nk, B_bound);
+  for (uint32_t pass = 0;; ++pass) {
+    PassCtl* cp = ctl + pass;
+    PassCtl* cn = ctl + pass + 1;
+    Range<K>* rc = pass == 0 ? rng_first : rng[pass & 1];
+    Range<K>* rn = rng[(pass + 1) & 1];
+    K* src = (pass & 1) ? bufA : bufB;  // input of pass >= 1
+    K* dst = (pass & 1) ? bufB : bufA;  // output of this pass's compaction
+    // tile -> first range table: read by this pass's streaming kernels, written
+    // by this pass's plan for the next pass (so it must not alias)
+    uint32_t* wgf_cur = (uint32_t*)P(bWgFirst) + (size_t)(pass & 1) * c.G_max;
+    uint32_t* wgf_next = (uint32_t*)P(bWgFirst) + (size_t)((pass + 1) & 1) * c.G_max;
+    const uint32_t NT = c.NT;
+    // pass-1 range parameters live in LDS unless that would push either
+    // pass-1 kernel past kPass1ParamsLds (then they are read from global memory)
+    uint32_t p1_lds = 0;
+    if (pass == 1 && !c.seg_first) {
+      size_t cnt = ((size_t)B_bound * 4 + 15) / 16 * 16 + pass1_map_bytes<K>(B0, R0, L2, R_bound);
+      size_t cmp = compact_lds_bytes(B_bound, U_slot_bound + 4) + pass1_map_bytes<K>(B0, R0, L2, R_bound);
+      p1_lds = std::max(cnt, cmp) <= kPass1ParamsLds ? 1u : 0u;
     }
+    // count
+    if (pass == 0) {
+      size_t lds = count_lds0<T>(c);
+      LDS_CHECK(count_lds0_total<T>(c));
+      // when the tables already allow only one workgroup per CU and a second
+      // histogram still fits, each workgroup counts two consecutive tiles
+      // (one row each) without a barrier between them, so its loads do not
+      // drain and restart at a tile boundary (2^28 fp32: 0.185 -> 0.175 ms)
+      const size_t hist2 = (size_t)c.B0_bound * 4;
+      const uint32_t tpw =
+          (count_lds0_total<T>(c) > kLdsOneWgPerCu && count_lds0_total<T>(c) + hist2 <= kLdsLimit) ? 2u : 1u;
+      if (tpw == 2) lds += hist2;
+      set_lds_attr((const void*)k_count0<T>, lds);
+      prof.begin(GGMS_KERNEL_COUNT0, (int)pass);
+      k_count0<T><<<(G + tpw - 1) / tpw, NT, lds, st>>>(d_vec, rc, (K*)P(bLut), cp, rows, tpw);
+      prof.end();
+    } else if (pass == 1 && !c.seg_first) {
+      size_t lds = ((size_t)B_bound * 4 + 15) / 16 * 16 + pass1_map_bytes<K>(B0, R0, L2, p1_lds ? R_bound : 0);
+      LDS_CHECK(lds);
+      set_lds_attr((const void*)k_count1<K>, lds);
+      prof.begin(GGMS_KERNEL_COUNTS, (int)pass);
+      k_count1<K><<<G, NT, lds, st>>>(src, ctl, (K*)P(bLut), rng_first, (uint64_t*)P(bRank0),
+                                      (MapParam<K>*)P(bParams1), p1_lds ? (uint32_t)lds : 0u, cp, rows);
+      prof.end();
+    } else {
+      size_t lds = (size_t)B_bound * 4;
+      LDS_CHECK(lds);
+      set_lds_attr((const void*)k_countS<K>, lds);
+      prof.begin(GGMS_KERNEL_COUNTS, (int)pass);
+      k_countS<K><<<G, NT, lds, st>>>(src, rc, wgf_cur, cp, rows);
+      prof.end();
+    }
+    HIP_TRY(hipGetLastError());
+    prof.begin(GGMS_KERNEL_COLSUM, (int)pass);
+    k_colsum<<<(B_bound + 63) / 64, 1024, 0, st>>>(rows, cp, totals);
+    prof.end();
+    HIP_TRY(hipGetLastError());
+    // plan
+    PlanArgs<K> pl = plan_args_common<K>(c, L, W, nk, d_out);
+    pl.ranges = rc;
+    pl.ctl = cp;
+    pl.ctl_next = cn;
+    pl.next_ranges = rn;
+    pl.slot_of_bucket = slot_tab[pass & 1];
+    pl.wg_first_next = wgf_next;
+    pl.force_finish = (pass + 1 >= c.max_passes) ? 1u : c.force_finish;
+    pl.finish_cap = (pass == 0 && c.one_pass) ? kOnePassFinishCap * c.fin_cap : c.fin_cap;
+    pl.merge_small = (pass == 0 && !c.seg_first) ? 1u : 0u;
+    pl.next_params = (pass == 0 && !c.seg_first) ? (MapParam<K>*)P(bParams1) : nullptr;
+    pl.rank_words = (pass == 0 && !c.seg_first) ? (uint64_t*)P(bRank0) : nullptr;
+    pl.mirror = dmirror;
+    pl.mirror_seq = dseq;
+    if (++ctx->mirror_seq == 0) ++ctx->mirror_seq;
+    pl.seq = ctx->mirror_seq;
+    pl.nan_out = nullptr;
+    plan_groups<K>(pl, L, W, pass == 0 && c.seg_first);
+    size_t lds_plan = plan_lds_bytes(B_bound, nk);
+    pl.lds_words = (uint32_t)(lds_plan / 4);
+    LDS_CHECK(lds_plan);
+    set_lds_attr((const void*)k_plan<T>, lds_plan);
+    prof.begin(GGMS_KERNEL_PLAN, (int)pass);
+    k_plan<T><<<1, 1024, lds_plan, st>>>(pl);
+    prof.end();
+    HIP_TRY(hipGetLastError());
+    // compaction
+    if (pass == 0 && c.seg_first) {
+      // every k-bucket into its own segment (the finish reads segments)
+      s = launch_segmented_first_pass<T>(c, L, W, d_vec, n, G, cp, pl, src, dst, st, prof);
+      if (s) return s;
+    } else if (pass == 0) {
+      // dynamic part: map parameters then the slot table (cell table is static LDS)
+      size_t lds = (size_t)R_bound * sizeof(MapParam<K>) + (size_t)B_bound * 2;
+      LDS_CHECK(lds + LutGeom<K>::bytes());
+      set_lds_attr((const void*)k_compact0<T>, lds);
+      prof.begin(GGMS_KERNEL_COMPACT0, (int)pass);
+      k_compact0<T><<<G, NT, lds, st>>>(d_vec, rc, (K*)P(bLut), cp, rows, pl.slot_of_bucket, pl.slot_bucket,
+                                        dst);
+      prof.end();
+    } else if (pass == 1 && !c.seg_first) {
+      size_t lds = compact_lds_bytes(B_bound, U_slot_bound + 4) + pass1_map_bytes<K>(B0, R0, L2, p1_lds ? R_bound : 0);
+      // one workgroup per CU: its writes scatter over every k-bucket segment,
+      // and twice the workgroups in flight keep twice the partial HBM lines
+      // open (measured 0.197 ms with two per CU, 0.154 ms with one)
+      lds = std::max<size_t>(lds, kLdsOneWgPerCu);
+      LDS_CHECK(lds);
+      set_lds_attr((const void*)k_compact1<K>, lds);
+      prof.begin(GGMS_KERNEL_COMPACTS, (int)pass);
+      k_compact1<K><<<G, NT, lds, st>>>(src, ctl, (K*)P(bLut), rng_first, (uint64_t*)P(bRank0),
+                                        (MapParam<K>*)P(bParams1), p1_lds ? (uint32_t)lds : 0u, cp, rows,
+                                        pl.slot_of_bucket, pl.slot_dst, pl.slot_bucket, dst);
+      prof.end();
+    } else {
+      size_t lds = compact_lds_bytes(B_bound, U_slot_bound + 4);
+      LDS_CHECK(lds);
+      set_lds_attr((const void*)k_compactS<K>, lds);
+      prof.begin(GGMS_KERNEL_COMPACTS, (int)pass);
+      k_compactS<K><<<G, NT, lds, st>>>(src, rc, wgf_cur, cp, rows, pl.slot_of_bucket,
+                                        pl.slot_dst, pl.slot_bucket, dst);
+      prof.end();
+    }
+    HIP_TRY(hipGetLastError());
+    // the next pass (and this pass's finish) is planned from the control
+    // blocks the plan kernel wrote to host memory, while the compaction
+    // runs.  The host polls the sequence word the plan writes after them:
+    // an event recorded between the plan and the compaction would make the
+    // GPU drain and publish at that point (~6 us idle before each compaction).
+    s = wait_mirror(hseq, pl.seq, st);
+    if (s) return s;
+    const PassCtl h = hmirror[0];
+    const PassCtl hn = hmirror[1];
+    // the iterative first pass hands every k-bucket to pass 1
+    if ((pass > 0 || c.seg_first) && h.U_small > 0) {
+      // every segment within a quarter of the capacity: half-size workgroups
+      // (512 threads, half the LDS) so twice as many run at once
+      const bool half = h.small_max <= c.fin_cap / 4;
+      // many small segments beside a few large ones: the large ones first
+      // (full workgroups), then the small ones in half-size workgroups
+      const uint32_t U_grp = h.U_small - h.U_wave - h.U_wide;
+      const bool split = !half && c.fin_cap / 4 >= kFinishSplitLen &&
+                         U_grp - std::min(h.U_fin_big, U_grp) >= kFinishSplitMinSegs;
+      prof.begin(GGMS_KERNEL_FINISH, (int)pass);
+      if (split) {
+        k_finish<T><<<fin_grid, 1024, fin_lds, st>>>(dst, cp, pl.small_start, pl.small_len, pl.small_klo,
+                                                     pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
+                                                     k_state, d_out, c.fin_cap, dflag, 1u);
+        k_finish<T><<<fin_grid, 512, fin_lds / 2, st>>>(dst, cp, pl.small_start, pl.small_len, pl.small_klo,
+                                                        pl.small_khi, pl.small_kstart, pl.small_order, klist, k_rank,
+                                                        k_state, d_out, c.fin_cap / 2, dflag, 2u);
+      } else {
+        k_finish<T><<<fin_grid, half ? 512 : 1024, half ? fin_lds / 2 : fin_lds, st>>>(
+            dst, cp, pl.small_start, pl.small_len, pl.small_klo, pl.small_khi, pl.small_kstart, pl.small_order,
+            klist, k_rank, k_state, d_out, half ? c.fin_cap / 2 : c.fin_cap, dflag);
+      }
+      if (h.U_wide > 0)
+        k_finish_wide<T><<<std::min<uint32_t>(h.U_wide, (uint32_t)ctx->cus), 1024, wide_lds, st>>>(
+            dst, src, cp, pl.small_start, pl.small_len, pl.small_klo, pl.small_khi, pl.small_kstart, pl.small_order,
+            klist, k_rank, k_state, d_out, c.fin_cap);
+      prof.end();
+      HIP_TRY(hipGetLastError());
+    }
+    if (pass == 0 && (*hbad || h.nan_count)) {
+      HIP_TRY(hipStreamSynchronize(st));
+      return *hbad ? GGMS_EINVAL : GGMS_ENAN;
+    }
+    if (pass == 0) {
+      B0 = h.B;
+      R0 = h.R;
+      L2 = h.l2_used;
+    }
+    if (pass < GGMS_MAX_PASS_STATS) {
+      stt.n_in[pass] = h.n;
+      stt.active[pass] = h.U;
+      stt.n_kept[pass] = (uint64_t)h.N_big + h.N_small;
+      stt.buckets[pass] = h.B;
+    }
+    stt.passes = pass + 1;
+    stt.finished_segments += h.U_small;
+    if (h.N_big == 0 || h.U_big == 0) break;
+    if (pass + 1 >= c.max_passes) {  // cannot happen: the last pass forces finishing
+      HIP_TRY(hipStreamSynchronize(st));
+      return GGMS_EDEVICE;
+    }
+    G = hn.G;
+    B_bound = std::max<uint32_t>(hn.B, 1);
+    R_bound = hn.R;
+    U_slot_bound = std::min<uint32_t>(nk, B_bound);
   }
   HIP_TRY(hipStreamSynchronize(st));
   if (!out_on_device) memcpy(out, hout, (size_t)nk * sizeof(T));

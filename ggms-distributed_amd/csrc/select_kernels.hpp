@@ -567,17 +567,18 @@ __device__ void bitonic_sort_shfl(K* s, uint32_t M) {
 
 // SHFL: the register-resident form (bitonic_sort_shfl) where it applies; it
 // holds 2 E keys per thread at its LDS stages, so kernels held to 64 VGPRs
-// pass false and keep the LDS-stage form.
-template <class K, bool SW = false, bool SHFL = true>
+// pass false and keep the LDS-stage form.  EMAX: the most keys a thread holds
+// in that form (32 spills a little, which only the sorts that need it pay).
+template <class K, bool SW = false, bool SHFL = true, uint32_t EMAX = 16>
 __device__ void bitonic_sort_lds(K* s, uint32_t M) {
   const uint32_t e = M / blockDim.x;
   if (M == e * blockDim.x &&
       (e == 4 || e == 8 || (e == 16 && (sizeof(K) <= 4 || SHFL)) ||
-       (e == 32 && (sizeof(K) == 2 || (sizeof(K) == 4 && SHFL))))) {
+       (e == 32 && (sizeof(K) == 2 || (EMAX >= 32 && sizeof(K) == 4 && SHFL))))) {
     if (SHFL && e == 4) bitonic_sort_shfl<K, 4>(s, M);
     else if (SHFL && e == 8) bitonic_sort_shfl<K, 8>(s, M);
     else if (SHFL && e == 16) bitonic_sort_shfl<K, 16>(s, M);
-    else if (SHFL && e == 32 && sizeof(K) == 4) bitonic_sort_shfl<K, 32>(s, M);
+    else if (SHFL && EMAX >= 32 && e == 32 && sizeof(K) == 4) bitonic_sort_shfl<K, 32>(s, M);
     else if (e == 4) bitonic_sort_lds_reg<K, 4, SW>(s, M);
     else if (e == 8) bitonic_sort_lds_reg<K, 8, SW>(s, M);
     else if (e == 16) bitonic_sort_lds_reg<K, 16, SW>(s, M);
@@ -2891,7 +2892,7 @@ __device__ __forceinline__ void select_count_first(uint32_t* hist, K key, uint32
 // segment; s is then read only for the later digits (not at all when the
 // first digit covers every varying bit).
 template <class K>
-__device__ void radix_select_multi(const K* __restrict__ s, uint32_t len, K klo, K khi, uint32_t q, SelectLds& L,
+__device__ __forceinline__ void radix_select_multi(const K* __restrict__ s, uint32_t len, K klo, K khi, uint32_t q, SelectLds& L,
                                    bool counted = false) {
   constexpr uint32_t kb = sizeof(K) * 8;
   const uint32_t vary = bitlen64((uint64_t)(klo ^ khi));
@@ -3145,7 +3146,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8)
     uint32_t st, len, q0, q1;
     K klo, khi;
   };
-  auto order_of = [&](uint32_t x) { return small_order ? small_order[x] : x; };
+  auto order_of = [&](uint32_t x) { return small_order[x]; };
   auto seg_of = [&](uint32_t j) {
     Seg g;
     g.st = small_start[j];
@@ -3331,7 +3332,7 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
   __shared__ RadixSortLds RL;
   const uint32_t U_small = ctl->U_small, U_wide = ctl->U_wide;
   for (uint32_t jj = U_small - U_wide + blockIdx.x; jj < U_small; jj += gridDim.x) {
-    const uint32_t j = small_order ? small_order[jj] : jj;
+    const uint32_t j = small_order[jj];
     const uint32_t st = small_start[j], len = small_len[j];
     const K klo = small_klo[j], khi = small_khi[j];
     const uint32_t q0 = small_kstart[j], q1 = small_kstart[j + 1];
@@ -3345,7 +3346,7 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
       const uint32_t M = pow2ceil_u32(len);
       for (uint32_t i = len + threadIdx.x; i < M; i += blockDim.x) s[i] = KeyMax<K>::v;
       __syncthreads();
-      bitonic_sort_lds<K>(s, M);
+      bitonic_sort_lds<K, false, true, 32>(s, M);
       for (uint32_t qq = q0 + threadIdx.x; qq < q1; qq += blockDim.x) {
         const uint32_t k = klist[qq];
         out[k] = KeyTraits<T>::dec(s[k_rank[k] - 1]);
@@ -3396,38 +3397,83 @@ __global__ void __launch_bounds__(1024) k_finish_wide(typename KeyTraits<T>::K* 
 }
 
 // ---------------------------------------------------------------------------
-// Tiny inputs (n <= finish capacity): one segment holding everything.
+// Tiny inputs (n <= finish_sort_cap): the whole call in one launch of one
+// workgroup.  The keys go to LDS; with many ks, or few keys, they are sorted
+// there in registers and read at every rank, else radix-selected (the sort of
+// 1024 4-byte keys takes 3 us and of 8192 16, the select's four digits 10 to
+// 15 whatever the length, so the line is kTinySortLen).  ks may be
+// host-visible memory.  flags: [0] and [2] cleared, [1] set when a k lies
+// outside [1, n] (never selected).  Bound by latency: the ks' and keys' round
+// trips, then the sort.  Three launches (setup, copy, finish) took 22 us of
+// kernels at 1000 keys and 9 ks, this 6.4 (call 36 -> 21).
 // ---------------------------------------------------------------------------
+constexpr uint32_t kTinySortLen = 4096;
+// LDS keys of a tiny call (the sort network's size)
+__host__ __device__ __forceinline__ uint32_t tiny_keys(uint32_t n) {
+  uint32_t m = 256;
+  while (m < n) m <<= 1;
+  return m;
+}
 template <class T>
-__global__ void k_tiny_setup(const T* __restrict__ x, uint32_t n, uint32_t nk, typename KeyTraits<T>::K* __restrict__ buf,
-                             uint32_t* __restrict__ k_rank, uint32_t* __restrict__ k_state,
-                             uint32_t* __restrict__ small_start, uint32_t* __restrict__ small_len,
-                             typename KeyTraits<T>::K* __restrict__ small_klo, typename KeyTraits<T>::K* __restrict__ small_khi,
-                             uint32_t* __restrict__ small_kstart, uint32_t* __restrict__ klist, PassCtl* ctl,
-                             uint32_t wide) {
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) buf[i] = KeyTraits<T>::enc(x[i]);
-  __shared__ uint32_t scratch[32];
-  uint32_t cnt = 0;
-  for (uint32_t k = threadIdx.x; k < nk; k += blockDim.x) cnt += (k_state[k] == kLive);
-  uint32_t tot;
-  uint32_t off = block_excl_scan_u32(cnt, scratch, &tot);
-  for (uint32_t k = threadIdx.x; k < nk; k += blockDim.x)
-    if (k_state[k] == kLive) {
-      klist[off++] = k;
-      k_state[k] = kSmall;
+__global__ void __launch_bounds__(1024) k_tiny(const T* __restrict__ x, uint32_t n, const uint32_t* __restrict__ ks,
+                                               uint32_t nk, T* __restrict__ out, uint32_t* __restrict__ k_state,
+                                               uint32_t* __restrict__ flags) {
+  using K = typename KeyTraits<T>::K;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ SelectLds L;
+  __shared__ uint32_t bad;
+  K* s = reinterpret_cast<K*>(smem);
+  const uint32_t t = threadIdx.x, nt = blockDim.x;
+  if (t == 0) bad = 0;
+  const uint32_t k0 = t < nk ? ks[t] : 1u;  // in flight beside the keys' reads
+  constexpr uint32_t U = 8;
+  for (uint32_t i0 = t; i0 < n; i0 += U * nt) {
+    T v[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) v[u] = x[i0 + u * nt < n ? i0 + u * nt : i0];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      if (i0 + u * nt < n) s[i0 + u * nt] = KeyTraits<T>::enc(v[u]);
+  }
+  const bool sorted = nk > kSelectMaxKs || n <= kTinySortLen;
+  const uint32_t M = tiny_keys(n);
+  if (sorted)
+    for (uint32_t i = n + t; i < M; i += nt) s[i] = KeyMax<K>::v;
+  __syncthreads();
+  if (k0 < 1 || k0 > n) bad = 1u;
+  if (sorted) {
+    bitonic_sort_lds<K, false, true, 32>(s, M);
+    for (uint32_t i = t; i < nk; i += nt) {
+      const uint32_t k = i == t ? k0 : ks[i];
+      if (k < 1 || k > n) bad = 1u;
+      else out[i] = KeyTraits<T>::dec(s[n - k]);
     }
-  if (threadIdx.x == 0) {
-    small_start[0] = 0;
-    small_len[0] = n;
-    small_klo[0] = 0;
-    small_khi[0] = KeyMax<typename KeyTraits<T>::K>::v;
-    small_kstart[0] = 0;
-    small_kstart[1] = tot;
-    ctl->U_small = 1;
-    ctl->U_big = 0;
-    ctl->N_big = 0;
-    ctl->U = 1;
-    ctl->U_wide = wide;
+  } else {
+    // the valid ks to the first threads
+    if (t < 64) {
+      const bool ok = t < nk && k0 >= 1 && k0 <= n;
+      const uint64_t m = wave_ballot(ok);
+      if (ok) {
+        L.kid[mask_below(m)] = t;
+        L.rank[mask_below(m)] = n - k0 + 1;
+      }
+      if (t == 0) L.ng = (uint32_t)__builtin_popcountll(m);
+    }
+    __syncthreads();
+    const uint32_t q = L.ng;
+    uint32_t kk = 0, kr = 0;
+    if (t < q) {
+      kk = L.kid[t];
+      kr = L.rank[t];
+    }
+    __syncthreads();  // read before finish_segment writes them
+    if (q) finish_segment<T, K>(s, n, (K)0, KeyMax<K>::v, (K)0, q, kk, kr, k_state, out, L);
+  }
+  __syncthreads();
+  if (t == 0) {
+    flags[0] = 0;
+    flags[1] = bad;
+    flags[2] = 0;
   }
 }
 
