@@ -134,7 +134,7 @@ __device__ __forceinline__ void batch_finish(BatchLds<typename KeyTraits<T>::K>&
     uint32_t M = pow2ceil_u32(len);
     for (uint32_t i = len + threadIdx.x; i < M; i += blockDim.x) L.A[i] = KeyMax<K>::v;
     __syncthreads();
-    bitonic_sort_lds<K, true, false>(L.A, M);
+    bitonic_sort_lds<K>(L.A, M);
     for (uint32_t j = j0 + threadIdx.x; j < j1; j += blockDim.x) out[L.Ko[j]] = KeyTraits<T>::dec(L.A[L.Kr[j] - 1]);
   }
   __syncthreads();
@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
       if (threadIdx.x == 0) a.status[p] = GGMS_EINVAL;
       continue;
     }
-    bitonic_sort_lds<uint64_t, true, false>(kp, M);
+    bitonic_sort_lds<uint64_t>(kp, M);
     for (uint32_t j = threadIdx.x; j < nk; j += blockDim.x) {
       L.Kr[j] = (uint32_t)(kp[j] >> 32);
       L.Ko[j] = kb + (uint32_t)(kp[j] & 0xFFFFFFFFu);
@@ -287,12 +287,28 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
     K* sA = scr[0] + base;
     K* sB = scr[1] + base;
 
+    // len keys at p into L.A; the vectors that hold them stay inside the scratch
+    // buffers, which are 256-byte aligned and sized in multiples of that
+    auto load_keys = [&](const K* p, uint32_t len) {
+      const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 15u) / (uint32_t)sizeof(K);
+      load_segment<K>(p - mis, mis, len, [&](uint32_t i, K key, bool in) {
+        if (in) L.A[i] = key;
+      });
+    };
+
     if (n <= FIN) {
-      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) L.A[i] = KT::enc(x[i]);
-      __syncthreads();
       bool nan = false;
-      if (KT::kFloat)
-        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) nan |= (L.A[i] < KT::kNegInf) | (L.A[i] > KT::kPosInf);
+      for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 8 * blockDim.x) {  // eight loads in flight
+        T v[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) v[u] = x[i0 + u * blockDim.x < n ? i0 + u * blockDim.x : i0];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) {
+          const K k = KT::enc(v[u]);
+          if (KT::kFloat) nan |= (k < KT::kNegInf) | (k > KT::kPosInf);
+          if (i0 + u * blockDim.x < n) L.A[i0 + u * blockDim.x] = k;
+        }
+      }
       if (nan) atomicOr(&s_flag, 1u);
       __syncthreads();
       if (s_flag) {
@@ -338,44 +354,56 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
       }
     }
     __syncthreads();
-    bitonic_sort_lds<K, true, false>(samp, Sp);
-    if (threadIdx.x == 0) {
-      // equal-quantile pivots, NaN / edge / one-key ranges as in the large-problem splitter
-      uint32_t R = 0;
-      auto emit = [&](K lo, uint32_t rq) {
-        L.starts[R] = lo;
-        L.req[R] = rq;
-        R++;
+    bitonic_sort_lds<K>(samp, Sp);
+    // equal-quantile pivots, NaN / edge / one-key ranges as in the large-problem
+    // splitter: thread j holds pivot j (P <= 64, one wave), and every run of
+    // equal pivots emits from its first, placed by a scan
+    if (threadIdx.x < 64) {
+      const uint32_t j = threadIdx.x, Q = P + 1;  // pivots 0 .. P: lane 63 may own two
+      const uint32_t share = NB / P > 0 ? NB / P : 1;
+      auto piv = [&](uint32_t i) { return samp[(uint32_t)(((uint64_t)i * (S - 1)) / P)]; };
+      auto emits = [&](uint32_t i, bool& one, bool& inner) {  // one-key range, range up to the next pivot value
+        one = inner = false;
+        if (i >= Q || (i > 0 && piv(i) == piv(i - 1))) return;
+        const K v = piv(i);
+        if (piv(P) == v) one = true;  // the last run
+        else if (piv(i + 1) != v) inner = true;
+        else {
+          one = true;
+          uint32_t e = i + 1;
+          while (piv(e) == v) ++e;
+          inner = (K)(piv(e) - v) >= 2;
+        }
       };
-      uint32_t share = NB / P > 0 ? NB / P : 1;
-      if (KT::kFloat) emit((K)0, 1);
-      K first = samp[0];
-      if (first > lowest) emit(lowest, 1);
-      K prev = first;
-      uint32_t run = 1;
-      bool open = false;
-      for (uint32_t j = 1; j <= P; ++j) {
-        uint32_t idx = (uint32_t)(((uint64_t)j * (S - 1)) / P);
-        K v = samp[idx];
-        if (v == prev) {
-          run++;
-          continue;
+      bool o0, n0, o1 = false, n1 = false;
+      emits(j, o0, n0);
+      if (j + 64 < Q) emits(j + 64, o1, n1);
+      const K first = samp[0], last = piv(P);
+      const uint32_t pre = (KT::kFloat ? 1u : 0u) + (first > lowest ? 1u : 0u);
+      const uint32_t c0 = (uint32_t)o0 + (uint32_t)n0, c1 = (uint32_t)o1 + (uint32_t)n1;
+      const uint32_t i0 = wave_incl_scan_u32(c0), i1 = wave_incl_scan_u32(c1);
+      const uint32_t tot0 = readlane_u32(i0, 63), tot = tot0 + readlane_u32(i1, 63);
+      auto emit = [&](uint32_t at, K v, bool one, bool inner) {
+        if (one) {
+          L.starts[at] = v;
+          L.req[at++] = 1;
         }
-        if (run > 1) {
-          emit(prev, 1);  // heavy value: its own one-key range
-          if ((K)(v - prev) >= 2) emit((K)(prev + 1), share);
-        } else {
-          emit(prev, share);
+        if (inner) {
+          L.starts[at] = one ? (K)(v + 1) : v;
+          L.req[at] = share;
         }
-        open = true;
-        prev = v;
-        run = 1;
+      };
+      if (c0) emit(pre + i0 - c0, piv(j), o0, n0);
+      if (c1) emit(pre + tot0 + i1 - c1, piv(j + 64), o1, n1);
+      if (j == 0) {
+        uint32_t r = 0;
+        if (KT::kFloat) { L.starts[r] = (K)0; L.req[r++] = 1; }
+        if (first > lowest) { L.starts[r] = lowest; L.req[r++] = 1; }
+        r = pre + tot;
+        if (last < highest) { L.starts[r] = (K)(last + 1); L.req[r++] = 1; }
+        if (KT::kFloat) { L.starts[r] = (K)(highest + 1); L.req[r++] = 1; }
+        s_n = r;
       }
-      (void)open;
-      emit(prev, 1);
-      if (prev < highest) emit((K)(prev + 1), 1);
-      if (KT::kFloat) emit((K)(highest + 1), 1);
-      s_n = R;
     }
     __syncthreads();
     const uint32_t R = s_n;
@@ -538,8 +566,7 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
           few &= c_j1[e] - c_j0[e] <= kWaveSelectMaxKs;
           tot += c_len[e++];
         }
-        const K* src = sA + c_reg[c];
-        for (uint32_t i = threadIdx.x; i < tot; i += blockDim.x) L.A[i] = src[i];
+        load_keys(sA + c_reg[c], tot);
         __syncthreads();
         if (e - c == 1) {
           batch_finish<T>(L, tot, (K)0, KeyMax<K>::v, c_j0[c], c_j1[c], out, hist256, bcast);
@@ -547,17 +574,25 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
           const uint32_t w = threadIdx.x >> 6, nw = blockDim.x >> 6;
           for (uint32_t q = c + w; q < e; q += nw) {
             const K* cs = L.A + (c_reg[q] - c_reg[c]);
-            for (uint32_t j = c_j0[q]; j < c_j1[q]; ++j) {
-              const K key = wave_radix_select<K>(cs, c_len[q], c_klo[q], c_khi[q], L.Kr[j], whist + w * 256, s_wbc[w]);
+            const uint32_t len = c_len[q], k0 = c_j0[q], k1 = c_j1[q];
+            auto rank = [&](uint32_t j) { return L.Kr[j]; };
+            auto put = [&](uint32_t j, K key) {
               if (lane_id() == 0) out[L.Ko[j]] = KeyTraits<T>::dec(key);
-            }
+            };
+            if (len <= 64) wave_sort_pick<K, 1>(cs, len, k0, k1, rank, put);
+            else if (len <= 128) wave_sort_pick<K, 2>(cs, len, k0, k1, rank, put);
+            else if (len <= 256) wave_sort_pick<K, 4>(cs, len, k0, k1, rank, put);
+            else if (len <= 512) wave_sort_pick<K, 8>(cs, len, k0, k1, rank, put);
+            else
+              for (uint32_t j = k0; j < k1; ++j)
+                put(j, wave_radix_select<K>(cs, len, c_klo[q], c_khi[q], L.Kr[j], whist + w * 256, s_wbc[w]));
           }
           __syncthreads();
         } else {
           const uint32_t M = pow2ceil_u32(tot);
           for (uint32_t i = tot + threadIdx.x; i < M; i += blockDim.x) L.A[i] = KeyMax<K>::v;
           __syncthreads();
-          bitonic_sort_lds<K, true, false>(L.A, M);
+          bitonic_sort_lds<K>(L.A, M);
           for (uint32_t q = c; q < e; ++q) {
             const uint32_t off = c_reg[q] - c_reg[c];
             for (uint32_t j = c_j0[q] + threadIdx.x; j < c_j1[q]; j += blockDim.x)
@@ -579,7 +614,7 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
       uint32_t next_sp = sp - 1;
       const K* src = (it.buf ? sB : sA) + it.region;
       if (it.len <= FIN) {
-        for (uint32_t i = threadIdx.x; i < it.len; i += blockDim.x) L.A[i] = src[i];
+        load_keys(src, it.len);
         __syncthreads();
         batch_finish<T>(L, it.len, it.klo, it.khi, it.j0, it.j1, out, hist256, bcast);
       } else {

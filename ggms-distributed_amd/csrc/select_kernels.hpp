@@ -565,6 +565,34 @@ __device__ void bitonic_sort_shfl(K* s, uint32_t M) {
   __syncthreads();
 }
 
+// One wave sorts the len <= 64 E keys at a (any address space) in its
+// registers and calls f(j, key of rank rank(j)) for j in [j0, j1), uniform over
+// the wave.  No LDS besides the reads, no barrier.
+template <class K, int E, class RankF, class F>
+__device__ __forceinline__ void wave_sort_pick(const K* a, uint32_t len, uint32_t j0, uint32_t j1, RankF&& rank, F&& f) {
+  const uint32_t l = lane_id();
+  K r[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const uint32_t at = (uint32_t)i * 64 + l;
+    r[i] = at < len ? a[at] : (K)~(K)0;
+  }
+  sort_regs<K, E>(r);
+  sort_lanes<K, E>(r);
+  for (uint32_t j = j0; j < j1; ++j) {
+    const uint32_t p = rank(j) - 1;  // lane p / E, register p % E
+    K v = r[0];
+#pragma unroll
+    for (int i = 1; i < E; ++i) v = p % E == (uint32_t)i ? r[i] : v;
+    K k;
+    if constexpr (sizeof(K) == 8)
+      k = ((K)readlane_u32((uint32_t)(v >> 32), p / E) << 32) | (K)readlane_u32((uint32_t)v, p / E);
+    else
+      k = (K)readlane_u32((uint32_t)v, p / E);
+    f(j, k);
+  }
+}
+
 // SHFL: the register-resident form (bitonic_sort_shfl) where it applies; it
 // holds 2 E keys per thread at its LDS stages, so kernels held to 64 VGPRs
 // pass false and keep the LDS-stage form.  EMAX: the most keys a thread holds
@@ -1183,150 +1211,85 @@ __device__ __forceinline__ K l2_entry(const K* starts, uint32_t r0, uint32_t r1,
 }
 
 // Two-level table of a range list given its sorted starts (in LDS; the ranges
-// partition the key space, starts[0] == 0, R <= 2047).  Called by a whole
-// workgroup; writes level 1 and the level-2 tables to g_lut and returns the
-// number of level-2 tables in use (same value in every thread).
+// partition the key space, starts[0] == 0, R <= 2047), over a window of the key
+// space: cell c covers [wbase + (c << wsh), wbase + ((c + 1) << wsh)) (wbase =
+// 0, wsh = S1: the top key bits, the whole key space).  A thread takes a run of
+// consecutive cells: one binary search for the range of the first, then a walk
+// along the starts, which most cells hold none of, and 16-byte stores.  A cell
+// with two or more starts gets a level-2 table of 64 sub-cells when its width
+// allows (wsh >= 6) and tables are left, else a search entry.  dst (global
+// memory or LDS, 16-byte aligned): level 1, then the level-2 tables.  Whole
+// workgroup; returns the level-2 tables in use (same value in every thread).
+// Bound by latency, like all of its kernel.  Before, every start was counted in
+// its cell and the counts scanned: 6.3 us of k_plan0, 17.5 us in the batched
+// kernel (two binary searches a cell); now 3.6 and 4.5.
 template <class K>
-__device__ uint32_t build_lut(const K* starts, uint32_t R, K* __restrict__ g_lut) {
+__device__ uint32_t build_lut(const K* starts, uint32_t R, K* __restrict__ dst, K wbase = 0,
+                              uint32_t wsh = LutGeom<K>::S1) {
   using G = LutGeom<K>;
-  __shared__ uint32_t tab_cell[G::L2TABLES];
-  __shared__ uint32_t scan_s[32];
-  const uint32_t nt = blockDim.x;
-  // level 1; multi-start cells are numbered in cell order for level-2 tables
-  uint32_t per = (G::L1CELLS + nt - 1) / nt;
-  uint32_t c0 = threadIdx.x * per, c1 = c0 + per < G::L1CELLS ? c0 + per : G::L1CELLS;
-  uint32_t nmulti = 0;
-  for (uint32_t c = c0; c < c1; ++c) {
-    K lo = (K)((K)c << G::S1), hi = (K)(lo + G::M1);
-    uint32_t r0 = last_start_le<K>(starts, 0, R - 1, lo);
-    uint32_t r1 = last_start_le<K>(starts, r0, R - 1, hi);
-    nmulti += r1 > r0 + 1;
-  }
-  uint32_t tot;
-  uint32_t t = block_excl_scan_u32(nmulti, scan_s, &tot);
-  for (uint32_t c = c0; c < c1; ++c) {
-    K lo = (K)((K)c << G::S1), hi = (K)(lo + G::M1);
-    uint32_t r0 = last_start_le<K>(starts, 0, R - 1, lo);
-    uint32_t r1 = last_start_le<K>(starts, r0, R - 1, hi);
-    K e;
-    if (r1 == r0) {
-      e = ((K)r0 << G::S1) | G::M1;
-    } else if (r1 == r0 + 1) {
-      e = ((K)r0 << G::S1) | (K)(starts[r1] - lo - 1);
-    } else if (t < G::L2TABLES) {
-      tab_cell[t] = c;
-      e = G::FLAG | G::TABLE | (K)t;
-      t++;
-    } else {
-      e = G::FLAG | (K)r0 | ((K)r1 << 11);
+  constexpr uint32_t C = G::L1CELLS, N = 16 / sizeof(K);
+  __shared__ uint32_t tab_cell[G::L2TABLES], tab_r[G::L2TABLES];  // a tabled cell, its first and last range
+  __shared__ uint32_t tabs;
+  const uint32_t nt = blockDim.x, t = threadIdx.x;
+  const K wmask = wsh >= G::S1 ? G::M1 : (K)(((K)1 << wsh) - 1);
+  const bool tables = wsh >= 6;
+  if (t == 0) tabs = 0;
+  __syncthreads();
+  const uint32_t per = ((C + nt - 1) / nt + N - 1) / N * N;
+  for (uint32_t c0 = t * per; c0 < C; c0 += nt * per) {
+    uint32_t r = last_start_le<K>(starts, 0, R - 1, (K)(wbase + ((K)c0 << wsh)));
+    K next = r + 1 < R ? starts[r + 1] : (K)0;  // the start after r, if any
+    for (uint32_t v = 0; v < per && c0 + v < C; v += N) {
+      K e[N];
+#pragma unroll
+      for (uint32_t u = 0; u < N; ++u) {
+        const uint32_t c = c0 + v + u;
+        const K lo = (K)(wbase + ((K)c << wsh)), hi = (K)(lo + wmask);
+        if (r + 1 < R && next == lo) {  // a start on the cell's low edge
+          ++r;
+          next = r + 1 < R ? starts[r + 1] : (K)0;
+        }
+        const uint32_t r0 = r;
+        const K first = next;
+        if (r + 1 < R && next <= hi) {
+          ++r;
+          next = r + 1 < R ? starts[r + 1] : (K)0;
+          if (r + 1 < R && next <= hi) {  // many starts: to the last of them
+            r = last_start_le<K>(starts, r + 1, R - 1, hi);
+            next = r + 1 < R ? starts[r + 1] : (K)0;
+          }
+        }
+        if (r == r0) {
+          e[u] = ((K)r0 << G::S1) | G::M1;
+        } else if (r == r0 + 1) {
+          e[u] = ((K)r0 << G::S1) | (K)(first - lo - 1);
+        } else {
+          const uint32_t tb = tables ? atomicAdd(&tabs, 1u) : G::L2TABLES;
+          if (tb < G::L2TABLES) {
+            tab_cell[tb] = c;
+            tab_r[tb] = r0 | (r << 16);
+            e[u] = G::FLAG | G::TABLE | (K)tb;
+          } else {
+            e[u] = G::FLAG | (K)r0 | ((K)r << 11);
+          }
+        }
+      }
+      uint4 q;
+      __builtin_memcpy(&q, e, 16);
+      *reinterpret_cast<uint4*>(dst + c0 + v) = q;
     }
-    g_lut[c] = e;
   }
   __syncthreads();
   // level 2: 64 sub-cells of each tabled cell
-  uint32_t used = tot < G::L2TABLES ? tot : G::L2TABLES;
-  for (uint32_t i = threadIdx.x; i < used * 64; i += nt) {
-    uint32_t tb = i >> 6, sub = i & 63;
-    uint32_t c = tab_cell[tb];
-    K lo = (K)(((K)c << G::S1) | ((K)sub << G::S2)), hi = (K)(lo + G::M2);
-    uint32_t r0 = last_start_le<K>(starts, 0, R - 1, lo);
-    uint32_t r1 = last_start_le<K>(starts, r0, R - 1, hi);
-    g_lut[G::L1CELLS + i] = l2_entry<K>(starts, r0, r1, lo);
-  }
-  return used;
-}
-
-// Same table as build_lut, with every level-1 cell decided in O(1) from
-// counts instead of two binary searches, over a window of the key space:
-// cell c covers [wbase + (c << wsh), wbase + ((c + 1) << wsh)) (wbase = 0,
-// wsh = S1: the top key bits, the whole key space).  Each range start inside
-// the window is counted in its cell (16-bit counters, two per word) or, when
-// it sits exactly on the cell's low edge, flagged in a bitmap; starts below
-// the window are counted once.  An exclusive scan of the per-cell totals then
-// gives, for cell c with P starts before it (below the window or in earlier
-// cells),
-//   r0 = P + edge(c) - 1 (last start <= the cell's low key),
-//   r1 = r0 + inside(c)  (last start <= the cell's high key).
-// A cell with two or more starts gets a level-2 table of 64 sub-cells when
-// its width allows (wsh >= 6) and tables are left, else a search entry.
-// cw: LDS scratch of lut_count_words<K>() words.  Returns the level-2 tables
-// in use (same value in every thread).
-template <class K> __host__ __device__ constexpr uint32_t lut_count_words() {
-  return LutGeom<K>::L1CELLS / 2 + LutGeom<K>::L1CELLS / 32;
-}
-template <class K>
-__device__ uint32_t build_lut_counted(const K* starts, uint32_t R, K* __restrict__ g_lut, uint32_t* cw,
-                                      K wbase = 0, uint32_t wsh = LutGeom<K>::S1) {
-  using G = LutGeom<K>;
-  constexpr uint32_t C = G::L1CELLS;
-  uint32_t* edge = cw + C / 2;
-  __shared__ uint32_t tab_cell[G::L2TABLES];
-  __shared__ uint32_t scan_s[32];
-  __shared__ uint32_t below_s;
-  const uint32_t nt = blockDim.x, t = threadIdx.x;
-  const K wmask = wsh >= G::S1 ? G::M1 : (K)(((K)1 << wsh) - 1);
-  const K wmax = wsh >= G::S1 ? (K)~(K)0 : (K)((((K)C) << wsh) - 1);
-  for (uint32_t i = t; i < lut_count_words<K>(); i += nt) cw[i] = 0;
-  if (t == 0) below_s = 0;
-  __syncthreads();
-  for (uint32_t r = t; r < R; r += nt) {
-    const K st = starts[r];
-    if (st < wbase) {
-      atomicAdd(&below_s, 1u);
-      continue;
-    }
-    const K d = (K)(st - wbase);
-    if (d > wmax) continue;  // above the window: in no cell
-    const uint32_t c = (uint32_t)(d >> wsh);
-    if (d & wmask) atomicAdd(&cw[c >> 1], 1u << (16 * (c & 1)));
-    else atomicOr(&edge[c >> 5], 1u << (c & 31));
-  }
-  __syncthreads();
-  auto inside = [&](uint32_t c) { return (cw[c >> 1] >> (16 * (c & 1))) & 0xFFFFu; };
-  auto on_edge = [&](uint32_t c) { return (edge[c >> 5] >> (c & 31)) & 1u; };
-  const uint32_t per = (C + nt - 1) / nt;
-  const uint32_t c0 = t * per, c1 = c0 + per < C ? c0 + per : C;
-  uint32_t nst = 0, nmulti = 0;
-  for (uint32_t c = c0; c < c1; ++c) {
-    const uint32_t k = inside(c);
-    nst += k + on_edge(c);
-    nmulti += k >= 2;
-  }
-  uint32_t tot;
-  const uint32_t ex = block_excl_scan_u32((nmulti << 16) | nst, scan_s, &tot);  // both fit 16 bits
-  uint32_t P = below_s + (ex & 0xFFFFu), tix = ex >> 16;
-  const bool tables = wsh >= 6;
-  for (uint32_t c = c0; c < c1; ++c) {
-    const uint32_t k = inside(c), a = on_edge(c);
-    const uint32_t r0 = P + a - 1, r1 = r0 + k;
-    const K lo = (K)(wbase + ((K)c << wsh));
-    K e;
-    if (k == 0) {
-      e = ((K)r0 << G::S1) | G::M1;
-    } else if (k == 1) {
-      e = ((K)r0 << G::S1) | (K)(starts[r1] - lo - 1);
-    } else if (tables && tix < G::L2TABLES) {
-      tab_cell[tix] = c;
-      e = G::FLAG | G::TABLE | (K)tix;
-      tix++;
-    } else {
-      e = G::FLAG | (K)r0 | ((K)r1 << 11);
-    }
-    g_lut[c] = e;
-    P += a + k;
-  }
-  __syncthreads();
-  // level 2: 64 sub-cells of each tabled cell (few: binary search)
-  const uint32_t nm = tables ? tot >> 16 : 0u;
-  const uint32_t used = nm < G::L2TABLES ? nm : G::L2TABLES;
+  const uint32_t used = tabs < G::L2TABLES ? tabs : G::L2TABLES;
   const uint32_t ssh = wsh - 6;
   for (uint32_t i = t; i < used * 64; i += nt) {
-    uint32_t tb = i >> 6, sub = i & 63;
-    uint32_t c = tab_cell[tb];
-    K lo = (K)(wbase + ((K)c << wsh) + ((K)sub << ssh)), hi = (K)(lo + (((K)1 << ssh) - 1));
-    uint32_t r0 = last_start_le<K>(starts, 0, R - 1, lo);
-    uint32_t r1 = last_start_le<K>(starts, r0, R - 1, hi);
-    g_lut[G::L1CELLS + i] = l2_entry<K>(starts, r0, r1, lo);
+    const uint32_t tb = i >> 6, sub = i & 63;
+    const K lo = (K)(wbase + ((K)tab_cell[tb] << wsh) + ((K)sub << ssh)), hi = (K)(lo + (((K)1 << ssh) - 1));
+    const uint32_t ra = tab_r[tb] & 0xFFFFu, rb = tab_r[tb] >> 16;
+    const uint32_t r0 = last_start_le<K>(starts, ra, rb, lo);
+    const uint32_t r1 = last_start_le<K>(starts, r0, rb, hi);
+    dst[C + i] = l2_entry<K>(starts, r0, r1, lo);
   }
   return used;
 }
