@@ -41,8 +41,12 @@ constexpr uint32_t kBatchNB = 8192;        // LDS histogram capacity
 constexpr uint32_t kBatchMaxPieces = 64;
 constexpr uint32_t kBatchMaxRanges = 2 * (kBatchMaxPieces + 1) + 6;
 constexpr uint32_t kBatchClasses = GGMS_BATCH_CLASSES;
-// a run of first-pass children whose every member has at most this many ks is
-// answered by per-wave radix selects instead of one sort of the whole run
+// first-pass children that one wave answers: sorted in its registers up to
+// kWaveSortLen keys, radix-selected up to kWaveSelectLen with at most
+// kWaveSelectMaxKs ks (a wave's select of 2048 keys takes about as long as the
+// workgroup's; a sort of 1024, 16 keys a lane, longer than its select)
+constexpr uint32_t kWaveSortLen = 512;
+constexpr uint32_t kWaveSelectLen = 2048;
 constexpr uint32_t kWaveSelectMaxKs = 8;
 
 template <class K> struct BatchItem {
@@ -512,96 +516,84 @@ __global__ void __launch_bounds__(1024) k_batch(BatchArgs a) {
       __threadfence_block();
       __syncthreads();
     }
-    // ---- first-pass children.  They sit in sA in bucket order, so their key
-    // intervals are disjoint and increasing: a run of consecutive small
-    // children is loaded as one batch; each k is then either radix-selected
-    // inside its child by one wave (every child of the run holds at most
-    // kWaveSelectMaxKs ks: the waves work on different children with no
-    // workgroup barrier) or read off one sort of the whole run at (child
-    // offset in the batch + rank in child).  Big children move to the front
-    // of the stack for re-bucketing.
+    // ---- first-pass children.  They sit in sA in bucket order, one behind the
+    // other: runs of them that fit the finish buffer are loaded together and
+    // each is answered by one wave, with no workgroup barrier: up to
+    // kWaveSortLen keys sorted in its registers, longer ones radix-selected per
+    // k.  The work stack keeps those a whole workgroup does better (longer than
+    // kWaveSelectLen) or must (k-dense, larger than the finish buffer).  Runs
+    // are found by binary search in the children's offsets and the stack's
+    // children by ballots: walking the table, one LDS read per child, was 40 of
+    // the 54 us a 32768-key problem's children took; now 15 us in all.
     {
       // child tables in the histogram's space (nkids <= kBatchMaxKs: 16 bytes
-      // per child always fit), key intervals behind them when they fit too;
-      // the wave histograms take the compaction cursors' and the k-bucket
-      // table's space (both free until the work stack)
+      // per child always fit); the wave histograms take the compaction cursors'
+      // and the k-bucket table's space (both free until the work stack)
       uint32_t* c_len = L.H;
       uint32_t* c_j0 = c_len + nkids;
       uint32_t* c_j1 = c_j0 + nkids;
       uint32_t* c_reg = c_j1 + nkids;
-      K* c_klo = reinterpret_cast<K*>(c_reg + nkids);
-      K* c_khi = c_klo + nkids;
-      const bool kfit = (size_t)nkids * (16 + 2 * sizeof(K)) <= (size_t)kBatchNB * 4;
       uint32_t* whist = L.cursor;  // 256 bins per wave
       static_assert(16 * kBatchMaxKs <= kBatchNB * 4, "child tables");
       static_assert(16 * 256 <= 2 * kBatchMaxKs, "wave histograms: cursor + runb");
-      for (uint32_t c = threadIdx.x; c < nkids; c += blockDim.x) {
-        const BatchItem<K> it = stack[c];
-        c_len[c] = it.len;
-        c_j0[c] = it.j0;
-        c_j1[c] = it.j1;
-        c_reg[c] = it.region;
-        if (kfit) {
-          c_klo[c] = it.klo;
-          c_khi[c] = it.khi;
+      __shared__ uint64_t s_later[kBatchMaxKs / 64];  // children for the work stack
+      auto later = [](uint32_t len, uint32_t nk) {
+        return len > kWaveSelectLen || (len > kWaveSortLen && nk > kWaveSelectMaxKs);
+      };
+      for (uint32_t c0 = 0; c0 < nkids; c0 += blockDim.x) {
+        const uint32_t c = c0 + threadIdx.x;
+        bool l = false;
+        if (c < nkids) {
+          const BatchItem<K> it = stack[c];
+          c_len[c] = it.len;
+          c_j0[c] = it.j0;
+          c_j1[c] = it.j1;
+          c_reg[c] = it.region;
+          l = later(it.len, it.j1 - it.j0);
         }
+        const uint64_t m = wave_ballot(l);
+        if (lane_id() == 0 && c < nkids) s_later[c >> 6] = m;
       }
       __syncthreads();
-      if (threadIdx.x == 0) {
-        uint32_t nbig = 0;
-        for (uint32_t c = 0; c < nkids; ++c)
-          if (c_len[c] > FIN) stack[nbig++] = stack[c];
-        s_sp = nbig;
+      const uint32_t w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+      for (uint32_t c = 0, e; c < nkids; c = e) {
+        e = c + 1;
+        if (c_len[c] > FIN) continue;
+        const uint32_t end = c_reg[c] + FIN;  // the run ends where its keys reach this
+        for (uint32_t hi = nkids; e < hi;) {
+          const uint32_t mid = (e + hi) >> 1;
+          if (c_reg[mid] + c_len[mid] <= end) e = mid + 1; else hi = mid;
+        }
+        load_keys(sA + c_reg[c], c_reg[e - 1] + c_len[e - 1] - c_reg[c]);
+        __syncthreads();
+        for (uint32_t q = c + w; q < e; q += nw) {
+          const uint32_t len = c_len[q], k0 = c_j0[q], k1 = c_j1[q];
+          if (later(len, k1 - k0)) continue;
+          const K* cs = L.A + (c_reg[q] - c_reg[c]);
+          auto rank = [&](uint32_t j) { return L.Kr[j]; };
+          auto put = [&](uint32_t j, K key) {
+            if (lane_id() == 0) out[L.Ko[j]] = KeyTraits<T>::dec(key);
+          };
+          if (len <= 64) wave_sort_pick<K, 1>(cs, len, k0, k1, rank, put);
+          else if (len <= 128) wave_sort_pick<K, 2>(cs, len, k0, k1, rank, put);
+          else if (len <= 256) wave_sort_pick<K, 4>(cs, len, k0, k1, rank, put);
+          else if (len <= kWaveSortLen) wave_sort_pick<K, kWaveSortLen / 64>(cs, len, k0, k1, rank, put);
+          else {
+            const K klo = stack[q].klo, khi = stack[q].khi;
+            for (uint32_t j = k0; j < k1; ++j)
+              put(j, wave_radix_select<K>(cs, len, klo, khi, L.Kr[j], whist + w * 256, s_wbc[w]));
+          }
+        }
+        __syncthreads();
+      }
+      if (threadIdx.x == 0) {  // in order, so an item is read before its place is taken
+        uint32_t n_later = 0;
+        for (uint32_t v = 0; v < (nkids + 63) / 64; ++v)
+          for (uint64_t m = s_later[v]; m; m &= m - 1)
+            stack[n_later++] = stack[v * 64 + (uint32_t)__builtin_ctzll(m)];
+        s_sp = n_later;
       }
       __threadfence_block();
-      uint32_t c = 0;
-      while (c < nkids) {  // every thread walks the same LDS table: uniform
-        if (c_len[c] > FIN) {
-          ++c;
-          continue;
-        }
-        uint32_t e = c, tot = 0;
-        bool few = kfit;
-        while (e < nkids && c_len[e] <= FIN && tot + c_len[e] <= FIN) {
-          few &= c_j1[e] - c_j0[e] <= kWaveSelectMaxKs;
-          tot += c_len[e++];
-        }
-        load_keys(sA + c_reg[c], tot);
-        __syncthreads();
-        if (e - c == 1) {
-          batch_finish<T>(L, tot, (K)0, KeyMax<K>::v, c_j0[c], c_j1[c], out, hist256, bcast);
-        } else if (few) {
-          const uint32_t w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-          for (uint32_t q = c + w; q < e; q += nw) {
-            const K* cs = L.A + (c_reg[q] - c_reg[c]);
-            const uint32_t len = c_len[q], k0 = c_j0[q], k1 = c_j1[q];
-            auto rank = [&](uint32_t j) { return L.Kr[j]; };
-            auto put = [&](uint32_t j, K key) {
-              if (lane_id() == 0) out[L.Ko[j]] = KeyTraits<T>::dec(key);
-            };
-            if (len <= 64) wave_sort_pick<K, 1>(cs, len, k0, k1, rank, put);
-            else if (len <= 128) wave_sort_pick<K, 2>(cs, len, k0, k1, rank, put);
-            else if (len <= 256) wave_sort_pick<K, 4>(cs, len, k0, k1, rank, put);
-            else if (len <= 512) wave_sort_pick<K, 8>(cs, len, k0, k1, rank, put);
-            else
-              for (uint32_t j = k0; j < k1; ++j)
-                put(j, wave_radix_select<K>(cs, len, c_klo[q], c_khi[q], L.Kr[j], whist + w * 256, s_wbc[w]));
-          }
-          __syncthreads();
-        } else {
-          const uint32_t M = pow2ceil_u32(tot);
-          for (uint32_t i = tot + threadIdx.x; i < M; i += blockDim.x) L.A[i] = KeyMax<K>::v;
-          __syncthreads();
-          bitonic_sort_lds<K>(L.A, M);
-          for (uint32_t q = c; q < e; ++q) {
-            const uint32_t off = c_reg[q] - c_reg[c];
-            for (uint32_t j = c_j0[q] + threadIdx.x; j < c_j1[q]; j += blockDim.x)
-              out[L.Ko[j]] = KeyTraits<T>::dec(L.A[off + L.Kr[j] - 1]);
-          }
-          __syncthreads();
-        }
-        c = e;
-      }
     }
     __syncthreads();
     // ---- work stack: finish small items, re-bucket large ones -----------------
