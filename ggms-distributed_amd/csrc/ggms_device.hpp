@@ -124,20 +124,32 @@ template <class K> GGMS_HD uint32_t map_off(K key, K lo, uint32_t sh, uint32_t m
   return mult ? (uint32_t)(((uint64_t)t * (uint64_t)mult) >> 32) : t;
 }
 
-// First key of bucket `off` of range r (off < r.nb); may exceed r.hi for an
-// empty trailing bucket.
-template <class K> GGMS_HD uint64_t bucket_first_key_off(const Range<K>& r, uint32_t off) {
+// x / m for x < 2^48, given inv = 1.0 / m: the rounded product is within one of
+// the quotient, and the remainder tells which way (the 64-bit integer division
+// is a hundred instructions).
+GGMS_HD uint64_t div_by(uint64_t x, uint32_t m, double inv) {
+  uint64_t q = (uint64_t)((double)x * inv);
+  const int64_t r = (int64_t)(x - q * (uint64_t)m);
+  if (r < 0) --q;
+  else if (r >= (int64_t)(uint64_t)m) ++q;
+  return q;
+}
+
+// First key of bucket `off` of range r (off < r.nb <= 2^15; inv = 1.0 / r.mult
+// unless the map is the identity); may exceed r.hi for an empty trailing bucket.
+template <class K> GGMS_HD uint64_t bucket_first_key_off(const Range<K>& r, uint32_t off, double inv) {
   if (r.mult == 0) return (uint64_t)off;
-  uint64_t t = (((uint64_t)off << 32) + (uint64_t)r.mult - 1ull) / (uint64_t)r.mult;
+  uint64_t t = div_by(((uint64_t)off << 32) + (uint64_t)r.mult - 1ull, r.mult, inv);
   return t << r.sh;  // offset from lo, < 2^64 since t <= 2^32
 }
 
 // Key interval [klo, khi] of bucket `off` of range r.  Returns false if empty.
 template <class K> GGMS_HD bool bucket_interval(const Range<K>& r, uint32_t off, K& klo, K& khi) {
   uint64_t w = (uint64_t)(r.hi - r.lo);
-  uint64_t a = bucket_first_key_off(r, off);
+  const double inv = r.mult ? 1.0 / (double)r.mult : 0.0;
+  uint64_t a = bucket_first_key_off(r, off, inv);
   if (a > w) return false;
-  uint64_t b = (off + 1 < r.nb) ? bucket_first_key_off(r, off + 1) : w + 1;  // exclusive, may be 2^64 for u64
+  uint64_t b = (off + 1 < r.nb) ? bucket_first_key_off(r, off + 1, inv) : w + 1;  // exclusive, may be 2^64 for u64
   uint64_t last = (off + 1 < r.nb) ? (b - 1) : w;
   if (last > w) last = w;
   if (off + 1 < r.nb && b == 0) last = w;  // wrapped: only possible when w == 2^64-1

@@ -281,11 +281,14 @@ enum Buf {
 };
 static_assert(bCount <= kMaxBuffers, "workspace layout table too small");
 
+// Room of the per-bucket tables: some past the last bucket, for 16-byte accesses.
+static size_t table_buckets(const Config& c) { return (std::max<size_t>(c.B0_bound, c.B_cap) + 64 + 7) / 8 * 8; }
+
 template <class T>
 static Layout make_layout(uint64_t n, uint32_t nk, const Config& c) {
   using K = typename KeyTraits<T>::K;
   size_t sz[bCount];
-  size_t Bm = std::max<size_t>(c.B0_bound, c.B_cap) + 64;
+  size_t Bm = table_buckets(c);
   size_t Rm = std::max<size_t>(c.R0_bound, Bm) + 64;
   size_t nkp = std::max<uint32_t>(nk, 1);
   const size_t nbuf = n;
@@ -407,6 +410,34 @@ static void set_lds_attr(const void* fn, size_t bytes) {
   do {                                                \
     if ((bytes) > kLdsLimit) return GGMS_ENOTSUP;     \
   } while (0)
+
+// The plan of a pass of at most B_bound buckets and R_bound ranges: kept in
+// registers for up to kPlanRegMaxKpt * 1024 ks (one k a thread up to 1024, whose
+// form issues an eighth as much), passed through global memory above, where its
+// tables no longer fit LDS.
+template <class T>
+static ggms_status launch_plan(PlanArgs<typename KeyTraits<T>::K>& pl, uint32_t B_bound, uint32_t R_bound, uint32_t nk,
+                               hipStream_t st, Prof& prof, int pass) {
+  size_t lds = plan_lds_bytes(B_bound, nk);
+  const uint32_t kpt = nk <= 1024 ? 1u : kPlanRegMaxKpt;
+  const bool reg = nk <= kpt * 1024 && B_bound <= kPlanRegMaxB &&
+                   plan_reg_lds_bytes(B_bound, R_bound, kpt) <= kLdsLimit;
+  const void* fn = (const void*)k_plan<T>;
+  if (reg) {
+    lds = plan_reg_lds_bytes(B_bound, R_bound, kpt);
+    fn = kpt == 1 ? (const void*)k_plan_reg<T, 1> : (const void*)k_plan_reg<T, kPlanRegMaxKpt>;
+  }
+  pl.lds_words = (uint32_t)(lds / 4);
+  if (lds > kLdsLimit) return GGMS_ENOTSUP;
+  set_lds_attr(fn, lds);
+  prof.begin(GGMS_KERNEL_PLAN, pass);
+  if (!reg) k_plan<T><<<1, 1024, lds, st>>>(pl);
+  else if (kpt == 1) k_plan_reg<T, 1><<<1, 1024, lds, st>>>(pl, B_bound, R_bound);
+  else k_plan_reg<T, kPlanRegMaxKpt><<<1, 1024, lds, st>>>(pl, B_bound, R_bound);
+  prof.end();
+  HIP_TRY(hipGetLastError());
+  return GGMS_OK;
+}
 
 // Arguments of the first-pass planning kernel (sampling, pivots, range table;
 // optionally the setup step).
@@ -575,7 +606,7 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
 
   PlanArgs<K> pl = plan_args_common<K>(c, L, W, nk, d_out);
   uint16_t* slot_tab[2] = {(uint16_t*)P(bSlotOfBucket),
-                           (uint16_t*)P(bSlotOfBucket) + (std::max<size_t>(c.B0_bound, c.B_cap) + 64)};
+                           (uint16_t*)P(bSlotOfBucket) + table_buckets(c)};
   const uint32_t NT = c.NT;
   const uint32_t Gn = c.G_max_next;
   const uint32_t U_slot_bound = std::min<uint32_t>(nk, std::max(c.B0_bound, c.B_cap));
@@ -634,14 +665,10 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
     pl.mirror = nullptr;
     pl.nan_out = pass == 0 ? flags + 2 : nullptr;
     plan_groups<K>(pl, L, W, pass == 0 && c.seg_first);
-    const size_t lds_plan = plan_lds_bytes(B_bound, nk);
-    pl.lds_words = (uint32_t)(lds_plan / 4);
-    LDS_CHECK(lds_plan);
-    set_lds_attr((const void*)k_plan<T>, lds_plan);
-    prof.begin(GGMS_KERNEL_PLAN, (int)pass);
-    k_plan<T><<<1, 1024, lds_plan, st>>>(pl);
-    prof.end();
-    HIP_TRY(hipGetLastError());
+    // later passes' ranges are the big k-buckets of the pass before: at most one per k
+    const uint32_t R_bound = pass == 0 ? c.R0_bound : U_slot_bound;
+    const ggms_status sp = launch_plan<T>(pl, B_bound, R_bound, nk, st, prof, (int)pass);
+    if (sp) return sp;
     // compaction
     if (pass == 0 && c.seg_first) {
       ggms_status s1 = launch_segmented_first_pass<T>(c, L, W, d_vec, n, G0, cp, pl, src, dst, st, prof);
@@ -898,7 +925,7 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
   uint32_t G = G0, B_bound = c.B0_bound, R_bound = c.R0_bound;
   uint32_t B0 = c.B0_bound, R0 = c.R0_bound, L2 = LutGeom<K>::L2TABLES;  // exact after pass 0
   uint16_t* slot_tab[2] = {(uint16_t*)P(bSlotOfBucket),
-                           (uint16_t*)P(bSlotOfBucket) + (std::max<size_t>(c.B0_bound, c.B_cap) + 64)};
+                           (uint16_t*)P(bSlotOfBucket) + table_buckets(c)};
   uint32_t U_slot_bound = std::min<uint32_t>(nk, B_bound);
   for (uint32_t pass = 0;; ++pass) {
     PassCtl* cp = ctl + pass;
@@ -976,14 +1003,8 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
     pl.seq = ctx->mirror_seq;
     pl.nan_out = nullptr;
     plan_groups<K>(pl, L, W, pass == 0 && c.seg_first);
-    size_t lds_plan = plan_lds_bytes(B_bound, nk);
-    pl.lds_words = (uint32_t)(lds_plan / 4);
-    LDS_CHECK(lds_plan);
-    set_lds_attr((const void*)k_plan<T>, lds_plan);
-    prof.begin(GGMS_KERNEL_PLAN, (int)pass);
-    k_plan<T><<<1, 1024, lds_plan, st>>>(pl);
-    prof.end();
-    HIP_TRY(hipGetLastError());
+    s = launch_plan<T>(pl, B_bound, R_bound, nk, st, prof, (int)pass);
+    if (s) return s;
     // compaction
     if (pass == 0 && c.seg_first) {
       // every k-bucket into its own segment (the finish reads segments)

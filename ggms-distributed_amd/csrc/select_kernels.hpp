@@ -24,6 +24,7 @@
 // copyElements_iterative :611-656, updatePivots_iterative :715-758,
 // generateBucketsandSlopes_iterative :404-477, generatePivots :1011-1054.
 #pragma once
+#include <cstddef>
 #include <type_traits>
 
 #include "ggms_device.hpp"
@@ -207,6 +208,45 @@ __device__ __forceinline__ void block_excl_scan_u32x4(const uint32_t (&v)[4], ui
     const uint32_t ws = wave_incl_scan_u32(mine);
     tot[i] = readlane_u32(ws, 63);
     off[i] = readlane_u32(ws - mine, wv) + inc[i] - v[i];
+  }
+}
+
+// N exclusive scans over C chunks of blockDim (1024) values each, chunk u's
+// before chunk u + 1's (thread t holds v[i][u] = value u * 1024 + t of scan i):
+// one pair of barriers.  Only the first `chunks` hold values (uniform).
+// scratch: >= N * C * 16 u32 of LDS, C at most 8.
+template <uint32_t N, uint32_t C>
+__device__ __forceinline__ void block_excl_scan_chunks(const uint32_t (&v)[N][C], uint32_t (&off)[N][C], uint32_t (&tot)[N],
+                                                       uint32_t chunks, uint32_t* scratch) {
+  const uint32_t lane = lane_id(), wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  uint32_t inc[N][C];
+#pragma unroll
+  for (uint32_t i = 0; i < N; ++i)
+#pragma unroll
+    for (uint32_t u = 0; u < C; ++u) inc[i][u] = u < chunks ? wave_incl_scan_u32(v[i][u]) : 0u;
+  __syncthreads();
+  if (lane == 63) {
+#pragma unroll
+    for (uint32_t i = 0; i < N; ++i)
+#pragma unroll
+      for (uint32_t u = 0; u < C; ++u) scratch[(i * C + u) * 16 + wv] = inc[i][u];
+  }
+  __syncthreads();
+  // the waves' totals of a scan, in chunk order: two a lane
+#pragma unroll
+  for (uint32_t i = 0; i < N; ++i) {
+    const uint32_t e = 2 * lane < C * 16 ? 2 * lane : 0u;
+    const uint32_t use = 0u - (uint32_t)(2 * lane < C * 16);
+    const uint32_t a = scratch[i * C * 16 + e] & use, b = scratch[i * C * 16 + e + 1] & use;
+    const uint32_t ws = wave_incl_scan_u32(a + b);
+    tot[i] = readlane_u32(ws, 63);
+#pragma unroll
+    for (uint32_t u = 0; u < C; ++u) {
+      if (u >= chunks) continue;
+      const uint32_t x = u * 16 + wv;
+      const uint32_t before = readlane_u32(ws - a - b, x >> 1) + (x & 1u ? readlane_u32(a, x >> 1) : 0u);
+      off[i][u] = before + inc[i][u] - v[i][u];
+    }
   }
 }
 
@@ -1983,6 +2023,425 @@ __global__ void __launch_bounds__(1024) k_plan(PlanArgs<typename KeyTraits<T>::K
       a.mirror[1] = *cn;
       __threadfence_system();  // the mirror reaches host memory before the sequence word
       *reinterpret_cast<volatile uint32_t*>(a.mirror_seq) = a.seq;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// k_plan_reg: k_plan for at most KPT * 1024 ks, one workgroup of 1024 threads.
+// A thread keeps its ks (KPT), its run of the histogram (up to 20 buckets) and
+// its active buckets (KPT, consecutive) in registers from phase to phase, all
+// global reads of a phase are issued together, and what threads hand each other
+// (prefix, active bits and list, slots, k counts) stays in LDS; k_plan passes
+// it through global memory, a round trip per phase.  Same results as k_plan.
+// Bound by latency: one round trip for histogram and ks, then some fifteen
+// barriers; with 8192 ks by the issue of eight of everything a thread.  101 ks
+// in 14563 buckets: 11.8 us (k_plan 17); 1001: 15.1 (24); 8192 in 1136 buckets:
+// 21.8 (26), in 8165 of 14563: 49.9 (87).
+//
+// LDS of the launch, in words: P / (slots, k counts) | range bases / list
+// starts | active bits, their prefix, rank bits, first slots | active list /
+// segment classes | a byte per bucket that holds a k (a store a k; an atomic
+// on its bit serialises when neighbouring ks share a word: 1024 buckets with
+// 8192 ks 5 us of the kernel).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kPlanRegMaxKpt = 8;      // ks a thread
+constexpr uint32_t kPlanRegMaxB = 20 * 1024;  // buckets: 20 a thread
+__host__ __device__ __forceinline__ uint32_t plan_reg_words_p(uint32_t B, uint32_t kpt) {
+  const uint32_t prefix = (B + 3) & ~3u, tables = ((B + 7) / 8) * 4 + kpt * 1024;
+  return prefix > tables ? prefix : tables;
+}
+__host__ __device__ __forceinline__ uint32_t plan_reg_words_r(uint32_t R, uint32_t kpt) {
+  return ((R > kpt * 1024 ? R : kpt * 1024) + 3) & ~3u;
+}
+// R: bound of this pass's ranges
+__host__ __device__ __forceinline__ size_t plan_reg_lds_bytes(uint32_t B, uint32_t R, uint32_t kpt) {
+  return ((size_t)plan_reg_words_p(B, kpt) + plan_reg_words_r(R, kpt) + 4 * ((rank_word_count(B) + 3) & ~3u)) * 4 +
+         (size_t)kpt * 2048 + (size_t)rank_word_count(B) * 32;
+}
+
+template <class T, uint32_t KPT>
+__global__ void __launch_bounds__(1024) k_plan_reg(PlanArgs<typename KeyTraits<T>::K> a, uint32_t B_bound,
+                                                   uint32_t R_bound) {
+  using K = typename KeyTraits<T>::K;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ uint32_t scratch[48 * KPT];
+  __shared__ uint32_t sh_max, sh_live, sh_fin_big, sh_wide, sh_wave;
+  __shared__ uint32_t ord_cnt[64];  // small segments per size class (kOrderBins used)
+  constexpr uint32_t nt = 1024;
+  const uint32_t t = threadIdx.x, lane = lane_id();
+  const PassCtl& ctl = *a.ctl;
+  const uint32_t n = ctl.n;
+  if (n == 0) return;
+  const uint32_t B = ctl.B, R = ctl.R, NW = rank_word_count(B);
+  uint32_t* P = reinterpret_cast<uint32_t*>(smem);
+  uint32_t* rbase = P + plan_reg_words_p(B_bound, KPT);
+  uint32_t* bits = rbase + plan_reg_words_r(R_bound, KPT);
+  const uint32_t NWp = (rank_word_count(B_bound) + 3) & ~3u;
+  uint32_t* wpre = bits + NWp;
+  uint32_t* rk_bits = wpre + NWp;
+  uint32_t* rk_first = rk_bits + NWp;
+  uint16_t* act = reinterpret_cast<uint16_t*>(rk_first + NWp);  // active buckets in order
+  uint4* flag4 = reinterpret_cast<uint4*>(act + KPT * 1024);    // 32 buckets' bytes: two of these
+  uint8_t* flag = reinterpret_cast<uint8_t*>(flag4);
+  // later uses of the same space
+  uint16_t* slot16 = reinterpret_cast<uint16_t*>(P);            // slot of every bucket
+  uint32_t* kfill = P + ((B + 7) / 8) * 4;                      // ks per small segment
+  uint32_t* kst = rbase;                                        // first k-list position of it
+  uint16_t* sinfo = act;                                        // its class information
+
+  // 0. ks, histogram and range bases
+  uint32_t st[KPT], rk[KPT], bk[KPT];
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    const uint32_t k = t + u * nt;
+    st[u] = k < a.nk ? a.k_state[k] : (uint32_t)kDone;
+    rk[u] = k < a.nk ? a.k_rank[k] : 0u;
+  }
+  const uint32_t per = ((B + nt - 1) / nt + 3) & ~3u;  // buckets a thread, at most 20
+  const uint32_t i0 = t * per;
+  uint4 tv[5];
+#pragma unroll
+  for (uint32_t q = 0; q < 5; ++q)  // the totals buffer has room past B
+    if (4 * q < per && i0 + 4 * q < B) tv[q] = *reinterpret_cast<const uint4*>(a.totals + i0 + 4 * q);
+  for (uint32_t r = t; r < R; r += nt) rbase[r] = a.ranges[r].base;
+  for (uint32_t w = t; w < NW; w += nt) {
+    flag4[2 * w] = make_uint4(0, 0, 0, 0);
+    flag4[2 * w + 1] = make_uint4(0, 0, 0, 0);
+    rk_bits[w] = 0;
+    rk_first[w] = kNone32;
+  }
+  uint32_t nan = 0, ctl_word = 0;
+  if (t < 64) {  // the first wave writes the control blocks
+    if (t < sizeof(PassCtl) / 4) ctl_word = reinterpret_cast<const uint32_t*>(a.ctl)[t];
+    ord_cnt[t] = 0;
+    sh_max = 0;
+    sh_live = 0;
+    if (ctl.nan_lo_bucket != kNone32) nan += a.totals[ctl.nan_lo_bucket];
+    if (ctl.nan_hi_bucket != kNone32) nan += a.totals[ctl.nan_hi_bucket];
+  }
+
+  // 1. inclusive prefix
+  uint32_t sum = 0;
+  auto each4 = [&](auto&& f) {
+#pragma unroll
+    for (uint32_t q = 0; q < 5; ++q)
+      if (4 * q < per && i0 + 4 * q < B) f(q, i0 + 4 * q);
+  };
+  each4([&](uint32_t q, uint32_t i) {
+    tv[q].y = i + 1 < B ? tv[q].y : 0u;
+    tv[q].z = i + 2 < B ? tv[q].z : 0u;
+    tv[q].w = i + 3 < B ? tv[q].w : 0u;
+    sum += tv[q].x + tv[q].y + tv[q].z + tv[q].w;
+  });
+  uint32_t tot;
+  uint32_t run = block_excl_scan_u32(sum, scratch, &tot);
+  each4([&](uint32_t q, uint32_t i) {
+    uint4 p;
+    p.x = run + tv[q].x;
+    p.y = p.x + tv[q].y;
+    p.z = p.y + tv[q].z;
+    p.w = p.z + tv[q].w;
+    run = p.w;
+    *reinterpret_cast<uint4*>(P + i) = p;
+  });
+  __syncthreads();
+
+  // 2. findKBuckets: the first bucket whose prefix reaches the rank, the steps
+  //    of a thread's searches interleaved (rank 0: not live, bucket 0)
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    rk[u] = st[u] == kLive ? rk[u] : 0u;
+    bk[u] = 0;
+  }
+  for (uint32_t len = B; len > 1;) {
+    const uint32_t half = len >> 1;
+    len -= half;
+#pragma unroll
+    for (uint32_t u = 0; u < KPT; ++u) bk[u] += P[bk[u] + half - 1] < rk[u] ? half : 0u;
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u)
+    if (st[u] == kLive) {
+      rk[u] -= bk[u] ? P[bk[u] - 1] : 0u;
+      flag[bk[u]] = 1;
+    }
+  __syncthreads();
+
+  // 3. number the active buckets in key order
+  uint32_t U;
+  {
+    const uint4 fa = flag4[2 * (t < NW ? t : NW - 1)], fb = flag4[2 * (t < NW ? t : NW - 1) + 1];
+    // four bytes of 0 or 1 to four bits
+    auto nib = [](uint32_t x) { return (x * 0x10204080u) >> 28; };
+    uint32_t word = nib(fa.x) | nib(fa.y) << 4 | nib(fa.z) << 8 | nib(fa.w) << 12 | nib(fb.x) << 16 | nib(fb.y) << 20 |
+                    nib(fb.z) << 24 | nib(fb.w) << 28;
+    word &= 0u - (uint32_t)(t < NW);
+    if (t < NW) bits[t] = word;
+    uint32_t off = block_excl_scan_u32((uint32_t)__builtin_popcount(word), scratch, &U);
+    if (t < NW) {
+      wpre[t] = off;
+      for (; word; word &= word - 1) act[off++] = (uint16_t)(t * 32 + (uint32_t)__builtin_ctz(word));
+    }
+  }
+  __syncthreads();
+
+  // 4. classify the active buckets (u * 1024 + t: this thread's); layout of the
+  //    next buffer: big segments first, then small ones
+  const uint32_t per_a = (U + nt - 1) / nt;  // of KPT
+  uint32_t ab[KPT], ac[KPT], cls[KPT], rg_of[KPT];
+  K klo[KPT], khi[KPT];
+  uint32_t sv[3][KPT], off[3][KPT], tots[3];  // big << 16 | small segments, their elements
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    const uint32_t q = u * nt + t;
+    ab[u] = q < U ? act[q] : 0u;
+    ac[u] = q < U ? P[ab[u]] - (ab[u] ? P[ab[u] - 1] : 0u) : 0u;
+    rg_of[u] = 0;
+  }
+  // owning range: the last with base <= b (rbase[0] == 0)
+  for (uint32_t len = R; len > 1;) {
+    const uint32_t half = len >> 1;
+    len -= half;
+#pragma unroll
+    for (uint32_t u = 0; u < KPT; ++u)
+      if (u < per_a) rg_of[u] += rbase[rg_of[u] + half] <= ab[u] ? half : 0u;
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    klo[u] = 0;
+    khi[u] = 0;
+    cls[u] = kResolved;
+    if (u < per_a && u * nt + t < U) {
+      const Range<K> rg = a.ranges[rg_of[u]];
+      bucket_interval<K>(rg, ab[u] - rg.base, klo[u], khi[u]);
+      if (klo[u] == khi[u]) a.act_klo[u * nt + t] = klo[u];
+      else cls[u] = a.merge_small || (ac[u] > a.finish_cap && !a.force_finish) ? kClsBig : kClsSmall;
+    }
+    sv[0][u] = cls[u] == kClsBig ? 0x10000u : cls[u] == kClsSmall ? 1u : 0u;
+    sv[1][u] = cls[u] == kClsBig ? ac[u] : 0u;
+    sv[2][u] = cls[u] == kClsSmall ? ac[u] : 0u;
+  }
+  static_assert(KPT * 1024 < 0x10000, "segment counts in 16 bits");
+  block_excl_scan_chunks<3, KPT>(sv, off, tots, per_a, scratch);
+  // (the prefix is read by now: its space holds the slots and the k counts)
+  const uint32_t U_big = tots[0] >> 16, U_small = tots[0] & 0xFFFFu, N_big = tots[1], N_small = tots[2];
+  for (uint32_t i = t; i < (B + 7) / 8; i += nt)
+    reinterpret_cast<uint4*>(slot16)[i] = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
+  for (uint32_t i = t; i < U_small; i += nt) kfill[i] = 0;
+
+  // 5. next pass's ranges: at least 2 buckets each when possible, the rest
+  //    proportional to the count; bucket bases by a scan
+  uint32_t Bn = a.B_req;
+  if (Bn < 4 * U_big) Bn = 4 * U_big;
+  if (Bn > a.B_cap) Bn = a.B_cap;
+  uint32_t nbv[1][KPT], nbase[1][KPT], nsh[KPT], nmult[KPT], B_next[1];
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    nbv[0][u] = 0;
+    if (cls[u] != kClsBig) continue;
+    Range<K> nr;
+    nr.lo = klo[u];
+    nr.hi = khi[u];
+    uint32_t nb;
+    if (2 * U_big <= Bn) nb = 2 + (uint32_t)(((uint64_t)ac[u] * (Bn - 2 * U_big)) / N_big);
+    else nb = 1 + (uint32_t)(((uint64_t)ac[u] * (Bn - U_big)) / N_big);
+    make_map<K>(nr, nb);
+    nbv[0][u] = nr.nb;
+    nsh[u] = nr.sh;
+    nmult[u] = nr.mult;
+  }
+  block_excl_scan_chunks<1, KPT>(nbv, nbase, B_next, per_a, scratch);
+
+  uint32_t Gn = 0, tile = 0;
+  if (N_big > 0) {
+    Gn = (N_big + a.min_tile - 1) / a.min_tile;
+    if (Gn > a.G_max) Gn = a.G_max;
+    if (Gn < 1) Gn = 1;
+    tile = (N_big + Gn - 1) / Gn;
+    tile = (tile + 63) & ~63u;
+    Gn = (N_big + tile - 1) / tile;
+  }
+  uint32_t small_max = 0;
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    if (u >= per_a || cls[u] == kResolved) continue;
+    const bool big = cls[u] == kClsBig;
+    const uint32_t b = ab[u], c = ac[u];
+    const uint32_t s = big ? off[0][u] >> 16 : U_big + (off[0][u] & 0xFFFFu);
+    const uint32_t dst = big ? off[1][u] : N_big + off[2][u];
+    slot16[b] = (uint16_t)s;
+    a.slot_dst[s] = dst;
+    a.slot_bucket[s] = b;
+    if (a.grp_cursor && s % kGroupSlots == 0) {  // a group of the grouped compaction starts at its first slot
+      a.grp_start[s / kGroupSlots] = dst;
+      a.grp_cursor[s / kGroupSlots] = dst;
+    }
+    if (a.rank_words) {
+      atomicOr(&rk_bits[b >> 5], 1u << (b & 31u));
+      atomicMin(&rk_first[b >> 5], s);
+    }
+    if (big) {
+      Range<K> nr;
+      nr.lo = klo[u];
+      nr.hi = khi[u];
+      nr.seg_start = dst;
+      nr.seg_end = dst + c;
+      nr.nb = nbv[0][u];
+      nr.sh = nsh[u];
+      nr.mult = nmult[u];
+      nr.base = nbase[0][u];
+      a.next_ranges[s] = nr;
+      if (a.next_params) a.next_params[s] = to_param<K>(nr);
+      const uint32_t w1 = (nr.seg_end + tile - 1) / tile;
+      for (uint32_t w = (dst + tile - 1) / tile; w < w1 && w < Gn; ++w) a.wg_first_next[w] = s;
+    } else {
+      const uint32_t j = s - U_big;
+      a.small_start[j] = dst;
+      a.small_len[j] = c;
+      a.small_klo[j] = klo[u];
+      a.small_khi[j] = khi[u];
+      small_max = c > small_max ? c : small_max;
+      sinfo[j] = (uint16_t)order_bin_info<K>(c, klo[u], khi[u], a.fin_cap);
+    }
+  }
+  if (t == 0 && a.grp_cursor) a.grp_start[(U_big + U_small + kGroupSlots - 1) / kGroupSlots] = N_big + N_small;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {  // one LDS atomic per wave
+    const uint32_t o = (uint32_t)__shfl_xor((int)small_max, d, 64);
+    small_max = o > small_max ? o : small_max;
+  }
+  if (lane == 0 && small_max) atomicMax(&sh_max, small_max);
+  __threadfence_block();
+  __syncthreads();
+
+  // 6. re-rank the live ks; the slot tables go out
+  T* out = reinterpret_cast<T*>(a.out);
+  uint32_t live = 0;
+  uint32_t sl[KPT], dd[KPT];
+  K kk[KPT];
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    sl[u] = kNone32;
+    if (st[u] != kLive) continue;
+    const uint32_t b = bk[u], s = slot16[b];
+    sl[u] = s;
+    if (s == kNone16)
+      kk[u] = a.act_klo[wpre[b >> 5] + (uint32_t)__builtin_popcount(bits[b >> 5] & ((1u << (b & 31u)) - 1u))];
+    else if (s < U_big) dd[u] = a.slot_dst[s];
+  }
+  for (uint32_t i = t; i < (B + 7) / 8; i += nt)  // the table has room past B
+    reinterpret_cast<uint4*>(a.slot_of_bucket)[i] = reinterpret_cast<const uint4*>(slot16)[i];
+  if (a.rank_words)
+    for (uint32_t w = t; w < NW; w += nt) {
+      const uint32_t b = rk_bits[w];
+      a.rank_words[w] = ((uint64_t)(b ? rk_first[w] : 0u) << 32) | b;
+    }
+  uint32_t kp[KPT];  // position in its segment's k list
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    if (st[u] != kLive) continue;
+    const uint32_t k = t + u * nt;
+    if (sl[u] == kNone16) {
+      out[k] = KeyTraits<T>::dec(kk[u]);
+      a.k_state[k] = kDone;
+    } else if (sl[u] < U_big) {
+      a.k_rank[k] = dd[u] + rk[u];
+      live++;
+    } else {
+      a.k_rank[k] = rk[u];
+      a.k_aux[k] = sl[u] - U_big;
+      a.k_state[k] = kSmall;
+      kp[u] = atomicAdd(&kfill[sl[u] - U_big], 1u);
+    }
+  }
+  const uint32_t wave_live = readlane_u32(wave_incl_scan_u32(live), 63);
+  if (lane == 0 && wave_live) atomicAdd(&sh_live, wave_live);
+  __syncthreads();
+
+  // 7. k lists and finish order of the small segments (largest class first)
+  const bool waves = U_small >= kFinishWaveMinSegs;
+  const uint32_t per_j = (U_small + nt - 1) / nt;  // segments u * 1024 + t, of KPT
+  uint32_t bin[KPT], nks[1][KPT], koff[1][KPT], ktot[1];
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    bin[u] = kNone32;
+    nks[0][u] = 0;
+    if (u >= per_j) continue;
+    const bool in = u * nt + t < U_small;
+    if (in) {
+      nks[0][u] = kfill[u * nt + t];
+      bin[u] = order_bin_of(sinfo[u * nt + t], nks[0][u], waves);
+    }
+    lds_count(ord_cnt, bin[u], in);
+  }
+  block_excl_scan_chunks<1, KPT>(nks, koff, ktot, per_j, scratch);
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u)
+    if (bin[u] != kNone32) {
+      a.small_kstart[u * nt + t] = koff[0][u];
+      kst[u * nt + t] = koff[0][u];
+    }
+  if (t < 64) {  // lane l: class kOrderBins - 1 - l
+    const uint32_t c = (kOrderBins - 1 - t) & 63u;  // the words past kOrderBins are zero
+    const uint32_t v = ord_cnt[c];
+    const uint32_t ex = wave_incl_scan_u32(v) - v;
+    ord_cnt[c] = ex;
+    if (t == kOrderBins - 1) sh_wide = v;
+    if (t == kOrderBins - 2) sh_wave = v;
+    // the classes from kFinishSplitLen keys up come first: they end where the class below them starts
+    if (t == kOrderBins - 1 - (2 + (kFinishSplitLen >> 10) - 1)) sh_fin_big = ex;
+    if (t == 0) a.small_kstart[U_small] = ktot[0];
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u)
+    if (st[u] == kLive && sl[u] != kNone16 && sl[u] >= U_big) a.klist[kst[sl[u] - U_big] + kp[u]] = t + u * nt;
+#pragma unroll
+  for (uint32_t u = 0; u < KPT; ++u) {
+    if (u >= per_j) continue;
+    const uint32_t pos = lds_claim(ord_cnt, bin[u], bin[u] != kNone32);
+    if (bin[u] != kNone32) a.small_order[pos] = u * nt + t;
+  }
+
+  // 8. control blocks, and their copy for the host: one word a lane, this
+  //    pass's in lanes 0 .. 31 and the next's in 32 .. 63
+  if (t < 64) {
+    constexpr uint32_t W = sizeof(PassCtl) / 4;
+    static_assert(W <= 32, "one word a lane, two blocks a wave");
+    uint32_t v = ctl_word;
+#define GGMS_PUT(block, field, value) v = lane == (block) * 32 + offsetof(PassCtl, field) / 4 ? (uint32_t)(value) : v
+    GGMS_PUT(0, U, U);
+    GGMS_PUT(0, U_big, U_big);
+    GGMS_PUT(0, U_small, U_small);
+    GGMS_PUT(0, U_slots, U_big + U_small);
+    GGMS_PUT(0, N_big, N_big);
+    GGMS_PUT(0, N_small, N_small);
+    GGMS_PUT(0, grp_sparse, (uint64_t)(N_big + N_small) * 4 < (uint64_t)n);
+    GGMS_PUT(0, live_ks, sh_live);
+    GGMS_PUT(0, U_wide, sh_wide);
+    GGMS_PUT(0, U_wave, sh_wave);
+    GGMS_PUT(0, U_fin_big, sh_fin_big);
+    GGMS_PUT(0, small_max, sh_max);
+    GGMS_PUT(0, nan_count, nan);
+    GGMS_PUT(1, n, N_big);
+    GGMS_PUT(1, tile, tile);
+    GGMS_PUT(1, G, Gn);
+    GGMS_PUT(1, R, U_big);
+    GGMS_PUT(1, Rp, pow2ceil_u32(U_big));
+    GGMS_PUT(1, B, B_next[0]);
+    GGMS_PUT(1, nan_lo_bucket, kNone32);
+    GGMS_PUT(1, nan_hi_bucket, kNone32);
+#undef GGMS_PUT
+    const uint32_t w = lane & 31u;
+    if (w < W) {
+      reinterpret_cast<uint32_t*>(lane < 32 ? const_cast<PassCtl*>(a.ctl) : a.ctl_next)[w] = v;
+      if (a.mirror) reinterpret_cast<uint32_t*>(a.mirror + (lane >> 5))[w] = v;
+    }
+    if (t == 0 && a.nan_out) *a.nan_out = nan;
+    if (a.mirror) {
+      __threadfence_system();  // the mirror reaches host memory before the sequence word
+      if (t == 0) *reinterpret_cast<volatile uint32_t*>(a.mirror_seq) = a.seq;
     }
   }
 }
