@@ -835,9 +835,13 @@ __device__ __forceinline__ void stream_tile(const V* __restrict__ x, uint32_t t0
 // loads, for data read from HBM exactly once (the caller's vector in the first
 // pass).  Later passes read what the previous compaction just wrote, much of
 // it still in the last-level cache, and lose with the hint (pass-1 compaction
-// 0.151 ms plain, 0.160 ms with it).  PIPE: the next four loads are issued
-// before the current four are processed (16 more VGPRs), for a workgroup that
-// streams alone on its CU and would otherwise leave HBM idle while it computes.
+// 0.151 ms plain, 0.160 ms with it).  PIPE: the next eight loads are issued
+// before the current eight are processed (48 more VGPRs), for a workgroup that
+// streams alone on its CU and would otherwise leave HBM idle while it computes:
+// the batched kernel, whose 16 waves a CU hold 128 KB in flight that way (4096
+// problems: 4.77 -> 4.58 ms against four).  The first-pass kernels lose with it
+// (count 177 -> 188 us, fp64 compaction 251 -> 258: two workgroups a CU, or
+// 256 that all stream at once, already keep HBM busy).
 template <class V, bool NT = false, bool PIPE = false, class FV, class F1>
 __device__ __forceinline__ void stream_tile_vec(const V* __restrict__ x, uint32_t t0, uint32_t t1, FV&& fv, F1&& f1) {
   constexpr int N = Vec16<V>::N;
@@ -846,20 +850,21 @@ __device__ __forceinline__ void stream_tile_vec(const V* __restrict__ x, uint32_
   uint32_t v1 = t1 / N;
   uint32_t v = t0 / N + threadIdx.x;
   if constexpr (PIPE) {
-    if (v + 3 * nt < v1) {
-      uint4 q[4];
+    constexpr uint32_t D = 8;
+    if (v + (D - 1) * nt < v1) {
+      uint4 q[D];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = NT ? ld_stream(xv + v + u * nt) : xv[v + u * nt];
+      for (uint32_t u = 0; u < D; ++u) q[u] = NT ? ld_stream(xv + v + u * nt) : xv[v + u * nt];
       for (;;) {
-        const uint32_t vn = v + 4 * nt;
-        const bool more = vn + 3 * nt < v1;
-        uint4 r[4];
+        const uint32_t vn = v + D * nt;
+        const bool more = vn + (D - 1) * nt < v1;
+        uint4 r[D];
         if (more) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) r[u] = NT ? ld_stream(xv + vn + u * nt) : xv[vn + u * nt];
+          for (uint32_t u = 0; u < D; ++u) r[u] = NT ? ld_stream(xv + vn + u * nt) : xv[vn + u * nt];
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (uint32_t u = 0; u < D; ++u) {
           V e[N];
           Vec16<V>::unpack(q[u], e);
           fv(e);
@@ -867,7 +872,7 @@ __device__ __forceinline__ void stream_tile_vec(const V* __restrict__ x, uint32_
         v = vn;
         if (!more) break;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) q[u] = r[u];
+        for (uint32_t u = 0; u < D; ++u) q[u] = r[u];
       }
     }
   }
