@@ -139,7 +139,9 @@ static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_o
   c.S = std::max<uint32_t>(8, std::min<uint32_t>(c.S, sizeof(K) == 4 ? 16384u : 8192u));
   uint32_t pieces = (c.mode == kModeLinear || c.mode == kModeStrided) ? std::max<uint32_t>(1, c.P - 1) : c.P;
   c.E = std::max<uint32_t>(1, c.B / pieces / 8);
-  uint32_t Q = (c.mode == kModeLinear || c.mode == kModeStrided) ? c.P : c.P + 1;
+  uint32_t Q = c.P + 1;
+  if (c.mode == kModeLinear || c.mode == kModeStrided)
+    Q = c.P > 3 && c.P - 1 <= kMaxRefinedPieces ? c.P + (kRefine - 1) * kMaxSplits : c.P;
   c.R0_bound = 2 * Q + 10;                // up to three edge ranges a side, and two for NaNs
   c.B0_bound = c.B + 2 * c.E + 8 + Q;
   c.NT = o.block_threads ? o.block_threads : 1024;

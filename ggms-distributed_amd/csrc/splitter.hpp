@@ -37,6 +37,11 @@ constexpr uint32_t kPlan0MaxRanges = 2064;
 // learned pivots are evaluated in chunks of this many (features of a chunk in LDS)
 constexpr uint32_t kMlpChunk = 128;
 constexpr uint32_t kMlpFeatStride = kMlpIn + 1;
+// linear splitter: a crowded piece is split into kRefine ranges, at most
+// kMaxSplits pieces of at most kMaxRefinedPieces (see k_plan0)
+constexpr uint32_t kRefine = 8, kMaxSplits = 4, kMaxRefinedPieces = 63;
+constexpr uint32_t kMaxRefinedPivots = kMaxRefinedPieces + 1 + (kRefine - 1) * kMaxSplits;
+constexpr float kCrowded = 0.4f;
 template <class K> __host__ __device__ constexpr size_t plan0_lds_bytes(uint32_t S_pad) {
   return (size_t)S_pad * sizeof(K) + 2048 * sizeof(K) + kPlan0MaxRanges * sizeof(K) +
          (kPlan0MaxRanges * 8 > (kMlpParams + kMlpChunk * kMlpFeatStride) * 4
@@ -263,29 +268,91 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
 
   // 2. pivots
   uint32_t Q = 0;
+  __shared__ uint32_t piece_w[kMaxRefinedPivots];  // weight of the range above each pivot, where pieces are split
+  __shared__ uint32_t refined_Q;
+  bool weights = false;
   if (a.mode == kModeLinear || a.mode == kModeStrided) {
     const uint32_t P = a.P;
     Q = P;
-    if (threadIdx.x == 0) {
-      if (P <= 3) {
-        q[0] = s[0];
-        if (P == 3) q[1] = s[S / 2];
-        q[P - 1] = s[S - 1];
-      } else {
-        uint32_t eo = (22u * S + 512u) / 1024u;
-        if (eo < 1) eo = 1;
-        if (2 * eo >= S) eo = S / 4 > 0 ? S / 4 : 1;
-        uint32_t po = (S - 2 * eo) / (P - 3);
-        q[0] = s[0];
-        q[1] = s[eo - 1];
-        for (uint32_t i = 2; i < P - 2; ++i) {
-          uint32_t idx = po * (i - 1) + eo - 1;
-          q[i] = s[idx < S ? idx : S - 1];
+    uint32_t eo = (22u * S + 512u) / 1024u;
+    if (eo < 1) eo = 1;
+    if (2 * eo >= S) eo = S / 4 > 0 ? S / 4 : 1;
+    const uint32_t po = P > 3 ? (S - 2 * eo) / (P - 3) : 0u;
+    auto at = [&](uint32_t i) {  // sample position of pivot i
+      if (i == 0) return 0u;
+      if (i == P - 1) return S - 1;
+      if (P == 3) return S / 2;
+      if (i == P - 2) return S - eo - 1;
+      const uint32_t x = po * (i - 1) + eo - 1;
+      return x < S ? x : S - 1;
+    };
+    weights = P > 3 && P - 1 <= kMaxRefinedPieces;
+    if (!weights) {
+      for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) q[i] = s[at(i)];
+    } else if (threadIdx.x < 64) {
+      // A piece whose sample crowds in part of its key span is split into
+      // kRefine ranges at its sample's quantiles, up to kMaxSplits of them (the
+      // most crowded first): keys are logarithmic, so around zero, or from zero
+      // up, a linear slope puts nearly the whole piece into its outermost
+      // buckets.  N(0,1), 16 pieces: the piece around zero is a sixteenth of the
+      // keys in a few buckets (2^28, 1001 ks: REFA M survivors of the first pass
+      // instead of 36.5 M).  Not the outermost pieces, a fiftieth of the sample
+      // each: their quantiles share cells of the cell table, whose slow path then
+      // costs every wave more than they save (count 180 -> 229 us).  Crowding: the sum of the squared shares
+      // of the four quarters of the span, 1/4 when even.
+      const uint32_t t = threadIdx.x;
+      const bool own = t < P - 1;
+      const uint32_t i0 = own ? at(t) : 0u, i1 = own ? at(t + 1) : 0u, n_in = i1 - i0;
+      const K lo = s[i0], span = (K)(s[i1] - lo);
+      float score = 0.0f;
+      if (own && n_in >= 4 * kRefine && n_in * 32 >= S && span >= (K)(8 * kRefine)) {
+        uint32_t prev = i0;
+        float sum = 0.0f;
+#pragma unroll
+        for (uint32_t quarter = 1; quarter <= 4; ++quarter) {
+          uint32_t x = i1;
+          if (quarter < 4) {  // first of the piece's samples at or above the quarter's end
+            const K end = (K)(lo + (span >> 2) * (K)quarter);
+            uint32_t l = prev;
+            while (l < x) {
+              const uint32_t mid = (l + x) >> 1;
+              if (s[mid] < end) l = mid + 1; else x = mid;
+            }
+          }
+          const float c = (float)(x - prev);
+          sum += c * c;
+          prev = x;
         }
-        q[P - 2] = s[S - eo - 1];
-        q[P - 1] = s[S - 1];
+        score = sum / ((float)n_in * (float)n_in);
+        if (score < kCrowded) score = 0.0f;
+      }
+      const uint32_t bits = __builtin_bit_cast(uint32_t, score);  // ordered as the scores: none is negative
+      uint32_t above = 0;
+      for (uint32_t l = 0; l < P - 1; ++l) {
+        const uint32_t o = readlane_u32(bits, l);
+        above += o > bits || (o == bits && l < t);
+      }
+      const bool split = bits != 0 && above < kMaxSplits;
+      const uint64_t m = wave_ballot(split);
+      if (own) {
+        const uint32_t first = t + (kRefine - 1) * mask_below(m);
+        q[first] = lo;
+        piece_w[first] = split ? 1u : kRefine;
+        if (split)
+          for (uint32_t j = 1; j < kRefine; ++j) {
+            q[first + j] = s[i0 + j * n_in / kRefine];
+            piece_w[first + j] = 1;
+          }
+      }
+      if (t == 0) {
+        const uint32_t n_q = P + (kRefine - 1) * (uint32_t)__builtin_popcountll(m);
+        q[n_q - 1] = s[S - 1];
+        piece_w[n_q - 1] = kRefine;
+        refined_Q = n_q;
       }
     }
+    __syncthreads();
+    if (weights) Q = refined_Q;
   } else {
     const uint32_t Pl = a.P;  // pieces
     Q = Pl + 1;
@@ -342,6 +409,7 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
     const EdgeCut<K> bot = edge_cut<K>((K)(q[0] - lowest), (K)(s[tail] - s[0]), a.E);
     const EdgeCut<K> top = edge_cut<K>((K)(highest - q[Q - 1]), (K)(s[S - 1] - s[S - 1 - tail]), a.E);
     const uint32_t pre = (KT::kFloat ? 1u : 0u) + bot.ranges();
+    auto weight = [&](uint32_t i) { return weights ? piece_w[i] : 1u; };
     const uint32_t per_q = (Q + blockDim.x - 1) / blockDim.x;
     const uint32_t i0 = threadIdx.x * per_q, i1 = i0 + per_q < Q ? i0 + per_q : Q;
     uint32_t cnt = 0, nint = 0;
@@ -353,13 +421,16 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
       if (j + 1 >= Q) cnt += 1;
       else if (j > i) {
         cnt += 1;
-        if ((K)(q[j + 1] - q[i]) >= 2) { cnt += 1; nint += 1; }
-      } else { cnt += 1; nint += 1; }
+        if ((K)(q[j + 1] - q[i]) >= 2) { cnt += 1; nint += weight(j); }
+      } else { cnt += 1; nint += weight(i); }
     }
-    uint32_t both;  // at most kPlan0MaxRanges of either: 16 bits each
+    uint32_t both;  // at most kPlan0MaxRanges ranges, and kRefine times the split pieces' pivots: 16 bits each
     uint32_t at = pre + (block_excl_scan_u32((nint << 16) | cnt, scan_tmp, &both) & 0xFFFFu);
     const uint32_t total = both & 0xFFFFu, ints = both >> 16;
-    const uint32_t share = ints ? (a.B / ints > 0 ? a.B / ints : 1u) : 1u;
+    auto share = [&](uint32_t i) {
+      const uint32_t x = a.B * weight(i) / ints;
+      return x > 0 ? x : 1u;
+    };
     for (uint32_t i = i0; i < i1; ++i) {
       if (i > 0 && q[i] == q[i - 1]) continue;
       const K v = q[i];
@@ -369,9 +440,9 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
         rlo[at] = v; rreq[at++] = 1;
       } else if (j > i) {
         rlo[at] = v; rreq[at++] = 1;
-        if ((K)(q[j + 1] - v) >= 2) { rlo[at] = (K)(v + 1); rreq[at++] = share; }
+        if ((K)(q[j + 1] - v) >= 2) { rlo[at] = (K)(v + 1); rreq[at++] = share(j); }
       } else {
-        rlo[at] = v; rreq[at++] = share;
+        rlo[at] = v; rreq[at++] = share(i);
       }
     }
     if (threadIdx.x == 0) {
