@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(1024) k_plan0(const T* __restrict__ x, Plan0Ar
       // most crowded first): keys are logarithmic, so around zero, or from zero
       // up, a linear slope puts nearly the whole piece into its outermost
       // buckets.  N(0,1), 16 pieces: the piece around zero is a sixteenth of the
-      // keys in a few buckets (2^28, 1001 ks: REFA M survivors of the first pass
+      // keys in a few buckets (2^28, 1001 ks: 22.9 M survivors of the first pass
       // instead of 36.5 M).  Not the outermost pieces, a fiftieth of the sample
       // each: their quantiles share cells of the cell table, whose slow path then
       // costs every wave more than they save (count 180 -> 229 us).  Crowding: the sum of the squared shares
