@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -64,6 +65,7 @@ struct Config {
   uint32_t min_tile;
   uint32_t max_passes;
   uint32_t fin_cap;
+  uint32_t finish_cap0;  // longest k-bucket of the first pass that goes straight to the finish
   uint64_t seed;
   uint32_t force_finish;
   bool one_pass;       // bucketMultiselect: one bucketing pass, every k-bucket finished
@@ -77,8 +79,30 @@ static uint32_t pow2ceil_host(uint32_t v) {
   return p;
 }
 
+// The ks fall into at most as many k-buckets as the first pass cuts from the
+// span of their ranks (those of a top-k call into a few).
+static uint32_t spread_of_ks(const uint32_t* ks, uint32_t nk, uint64_t n) {
+  const auto mm = std::minmax_element(ks, ks + nk);
+  return (uint32_t)std::min<uint64_t>(nk, (uint64_t)(*mm.second - *mm.first) * 14336u / n + 2);
+}
+
+// The one-pass bucketMultiselect of few ks finishes after its bucketing pass every
+// k-bucket of up to this many times the LDS capacity (the larger ones from
+// global memory); only k-buckets above that are re-bucketed first.
+constexpr uint32_t kOnePassFinishCap = 4;
+
+// With more ks than this the one-pass form keeps the full bucket count and
+// re-buckets every k-bucket above the LDS capacity: the finish reads a k-bucket
+// from global memory again for each group of its ks (2^24 fp32 N(0,1) with 2048
+// ks: 1198 us with those above it finished there, 272 re-bucketed; with 101 ks
+// at 2^22 it is the other way round, 109 against 127).
+constexpr uint32_t kOnePassFewKs = 256;
+
+// nk_spread: about how many buckets the ks fall into (0 = the full bucket
+// count, as for sizes that must hold for every call)
 template <class K>
-static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_opts& o, int cus) {
+static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_opts& o, int cus,
+                             uint32_t nk_spread = 0) {
   Config c{};
   c.mode = kModeLinear;
   if (alg == GGMS_ALG_DISTRIBUTED_1GPU || alg == GGMS_ALG_DISTRIBUTED_BUCKET_1GPU) c.mode = kModeStrided;
@@ -117,7 +141,25 @@ static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_o
   // 1.701 (one tile per CU makes the headline, 2^28 with 1001 ks, 0.68 -> 0.84
   // ms and |N(0,1)| at 2^26 0.655 -> 0.679).
   const bool big_seg = c.seg_first && !c.one_pass && n >= (1ull << 27);
-  c.B = o.num_buckets ? o.num_buckets : (big_seg ? 16384u : 14336u);
+  // Few ks or few keys take fewer buckets: the keys of the k-buckets are handled
+  // again (nk n / B of them) and every bucket costs the histogram rows, their
+  // sums and the plan, so the best count goes with the root of nk n.  A call at
+  // 14336 / 4096 buckets, in us: fp32 N(0,1) 2^20 with 101 ks 113 / 103, 2^22
+  // with 101 137 / 111, 2^24 with 301 (uniform) 181 / 160, 2^28 with 5 481 / 462,
+  // mixture 2^22 with 101 177 / 147 (sketch 194 / 166); past the line 2^24 with
+  // 2048 ks 232 / 240, 2^26 with 1001 267 / 321.  8-byte keys have it lower: fp64
+  // N(0,1) 2^22 with 101 146 / 131, with 1001 174 / 204.  The one-pass form
+  // finishes every k-bucket as the first pass left it: 2^22 with 101 125 / 109,
+  // top 1024 of 10^7 133 / 107, past its line 2^26 with 101 202 / 233.  Fewer
+  // than 4096 are no faster (2048, mixture 2^22 with 101, sketch: 208) and the
+  // iterative segmented form wants the full count (2^20 with 8192 ks 188 / 265).
+  uint32_t B_few = 14336u;
+  if (nk_spread && (c.one_pass ? nk_spread <= kOnePassFewKs : !c.seg_first)) {
+    const double w = c.one_pass ? 0.2 : sizeof(K) == 4 ? 0.05 : 0.15;
+    const double x = w * std::sqrt((double)nk_spread * (double)n);
+    B_few = x < 5800 ? 4096u : x < 8000 ? 8192u : 14336u;
+  }
+  c.B = o.num_buckets ? o.num_buckets : (big_seg ? 16384u : B_few);
   c.B = std::max<uint32_t>(16, std::min<uint32_t>(c.B, kMaxBuckets));
   c.B_cap = kMaxBuckets;
   if (c.mode == kModeLinear || c.mode == kModeStrided) {
@@ -159,9 +201,9 @@ static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_o
   if (c.device_schedule) c.max_passes = o.device_passes ? std::min<uint32_t>(o.device_passes, 8) : 3;
   if (c.max_passes < 2) c.max_passes = 2;  // the first pass always hands its k-buckets to a second
   c.fin_cap = sizeof(K) == 4 ? 32768 : 16384;  // 128 KB of LDS in the finishing kernel
+  c.finish_cap0 = c.one_pass && nk <= kOnePassFewKs ? kOnePassFinishCap * c.fin_cap : c.fin_cap;
   c.seed = o.seed;
   c.force_finish = 0;
-  (void)n;
   return c;
 }
 
@@ -355,11 +397,6 @@ static size_t count_lds0_total(const Config& c) {
   using K = typename KeyTraits<T>::K;
   return count_lds0<T>(c) + LutGeom<K>::bytes();
 }
-
-// The one-pass bucketMultiselect finishes after its bucketing pass every
-// k-bucket of up to this many times the LDS capacity (the larger ones from
-// global memory); only k-buckets above that are re-bucketed first.
-constexpr uint32_t kOnePassFinishCap = 4;
 
 // at most this many ks: the setup runs inside the first-pass planning kernel
 constexpr uint32_t kSetupInPlan0MaxKs = kSetupKsPerThread * 1024;
@@ -660,7 +697,7 @@ static ggms_status launch_fixed(const Config& c, const Layout& L, char* W, uint3
     pl.slot_of_bucket = slot_tab[pass & 1];
     pl.wg_first_next = (uint32_t*)P(bWgFirst) + (size_t)((pass + 1) & 1) * c.G_max;
     pl.force_finish = (pass + 1 >= passes) ? 1u : 0u;
-    pl.finish_cap = (pass == 0 && c.one_pass) ? kOnePassFinishCap * c.fin_cap : c.fin_cap;
+    if (pass == 0) pl.finish_cap = c.finish_cap0;
     pl.merge_small = (pass == 0 && !c.seg_first) ? 1u : 0u;
     pl.next_params = (pass == 0 && !c.seg_first) ? (MapParam<K>*)P(bParams1) : nullptr;
     pl.rank_words = (pass == 0 && !c.seg_first) ? (uint64_t*)P(bRank0) : nullptr;
@@ -802,7 +839,8 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
   if (!d_vec || !ks || !out) return GGMS_EINVAL;
   const uint32_t n = (uint32_t)n64;
   hipStream_t st = (hipStream_t)o.stream;
-  Config c = resolve_config<K>(alg, n64, nk, o, ctx->cus);
+  const uint32_t spread = ks_on_device ? nk : spread_of_ks(ks, nk, n64);
+  Config c = resolve_config<K>(alg, n64, nk, o, ctx->cus, spread);
   if (c.mode == kModeLearned && !learned_weights_device(ctx->device)) return GGMS_ENOTSUP;
   if (!ks_on_device)
     for (uint32_t i = 0; i < nk; ++i)
@@ -995,7 +1033,7 @@ static ggms_status run_select(ggms_ctx* ctx, ggms_alg alg, const T* d_vec, uint6
     pl.slot_of_bucket = slot_tab[pass & 1];
     pl.wg_first_next = wgf_next;
     pl.force_finish = (pass + 1 >= c.max_passes) ? 1u : c.force_finish;
-    pl.finish_cap = (pass == 0 && c.one_pass) ? kOnePassFinishCap * c.fin_cap : c.fin_cap;
+    if (pass == 0) pl.finish_cap = c.finish_cap0;
     pl.merge_small = (pass == 0 && !c.seg_first) ? 1u : 0u;
     pl.next_params = (pass == 0 && !c.seg_first) ? (MapParam<K>*)P(bParams1) : nullptr;
     pl.rank_words = (pass == 0 && !c.seg_first) ? (uint64_t*)P(bRank0) : nullptr;
@@ -1300,7 +1338,7 @@ static ggms_status run_noalloc(ggms_alg alg, const T* d_vec, uint64_t n64, const
   if (cus <= 0) cus = 256;
   ggms_opts od = o;
   od.schedule = GGMS_SCHEDULE_DEVICE;
-  const Config c = resolve_config<K>(alg, n64, nk, od, cus);
+  const Config c = resolve_config<K>(alg, n64, nk, od, cus, nk);
   if (c.mode == kModeLearned && !learned_weights_device(device)) return GGMS_ENOTSUP;
   const Layout L = make_layout<T>(n64, nk, c);
   // the status words sit behind the workspace

@@ -57,7 +57,7 @@ typedef enum {
 
 /* Tunables.  Zero means "library default" for every numeric field. */
 typedef struct {
-  uint32_t num_buckets;   /* buckets per pass (0 = auto: 14336, or 16384 when the first pass is segmented and n >= 2^27; max 16384; the reference uses 8192) */
+  uint32_t num_buckets;   /* buckets per pass (0 = auto: 14336, 16384 when the first pass is segmented and n >= 2^27, fewer, down to 4096, for calls of few keys or few ks; max 16384; the reference uses 8192) */
   uint32_t num_pivots;    /* linear splitter pivots (default 17 => 16 ranges) */
   uint32_t sample_size;   /* splitter sample (default 1024, 2048 for the linear splitter on 4-byte keys with n >= 2^27 and few ks; 8192 for the one-GPU distributed form) */
   uint32_t block_threads; /* workgroup size of the streaming kernels (default 1024) */
