@@ -956,17 +956,27 @@ __device__ __forceinline__ void stream_tile_any(const V* __restrict__ x, uint32_
 // start inside the cell, so the range of a key is
 //     r0 + ((key & cell_mask) > start_offset - 1)
 // with no branch.  A cell holding two or more starts points to a level-2
-// table of 64 sub-cells (next 6 key bits) in the same leaf format; when the
-// level-2 budget is used up, or a sub-cell still holds two or more starts,
-// the entry says "search" and carries the first/last candidate range for a
-// short binary search.  Both rarer paths sit behind wave-uniform tests.
+// table of 64 sub-cells (next 6 key bits) in the same leaf format, and a
+// sub-cell still holding two or more to a level-3 table of 64 cells between the
+// first and the last of them; when the tables are used up, or a cell of level 3
+// holds several, the entry says "search" and carries the first/last candidate
+// range for a short binary search.  The rarer paths sit behind wave-uniform tests.
 //
 // Entry layout (E = K: 32-bit entries for u32 keys, 64-bit for u64 keys;
 // KB = key bits, S1 = KB - level-1 bits, S2 = S1 - 6):
 //   level-1 leaf:   bit KB-1 = 0 | r0 in bits [S1, S1+11) | start_offset-1 in bits [0, S1)
 //   level-2 leaf:   bit KB-1 = 0 | r0 in bits [S2, S2+17) | start_offset-1 in bits [0, S2)
 //   level-1 table:  bit KB-1 = 1, bit KB-2 = 1 | table index
-//   search (1, 2):  bit KB-1 = 1, bit KB-2 = 0 | r0 in bits [0, 11) | r1 in bits [11, 22)
+//   search:         bit KB-1 = 1, bit KB-2 = 0 | r0 in bits [0, 11) | r1 in bits [11, 22)
+//   level-3 table:  bit KB-1 = 1, bit KB-2 = 0, bit 22 | r0 in bits [0, 11) | shift in [11, 17) | table in [23, 29)
+// A level-2 sub-cell with two or more starts gets one of the tables the cells
+// left over, as level 3: 64 cells of 2^shift keys from its first inside start on
+// (a key below that is of range r0; the last cell holds no start and stands for
+// all keys past it), with the entries of level 2.  A search is a read of LDS and
+// a handful of instructions a step for the whole wave, whichever lanes need it:
+// the components of a mixture that are narrow beside their distance from zero
+// put 16 ranges and a tenth of the keys into one sub-cell (2^28 keys, 8192 ks:
+// first-pass count 570 -> 413 us, compaction 1118 -> 955, mean of nine mixtures).
 // The map parameters of a range are packed for one 16-byte (u32 keys) or
 // 32-byte (u64 keys) LDS read.
 // ---------------------------------------------------------------------------
@@ -989,9 +999,13 @@ template <class K> struct LutGeom {
   static constexpr uint32_t L1CELLS = 1u << L1BITS;
   static constexpr uint32_t S1 = KB - L1BITS;
   static constexpr uint32_t S2 = S1 - 6;
-  static constexpr uint32_t L2TABLES = 32u;  // 8 KB (u32) / 16 KB (u64) of level 2
+  // 10 KB (u32) / 16 KB (u64) of levels 2 and 3.  At 32 the tables of u32 ran
+  // out on one of ten mixtures (2^28 keys 1.87 -> 2.20 ms); 44 and 48 cost the
+  // first-pass count of every input its room in LDS (2^28 N(0,1) 185 -> 191 us).
+  static constexpr uint32_t L2TABLES = sizeof(K) == 4 ? 40u : 32u;
   static constexpr K FLAG = (K)1 << (KB - 1);
   static constexpr K TABLE = (K)1 << (KB - 2);
+  static constexpr K DEEP = (K)1 << 22;
   static constexpr K M1 = ((K)1 << S1) - 1;
   static constexpr K M2 = ((K)1 << S2) - 1;
   static __host__ __device__ constexpr size_t bytes() { return (size_t)(L1CELLS + L2TABLES * 64) * sizeof(K); }
@@ -1165,6 +1179,18 @@ template <class K> struct Pass0Map {
     r = (uint32_t)((e2 >> G::S2) & 0x1FFFF) + (soff > (e2 & G::M2) ? 1u : 0u);
     return e2;
   }
+  // level3: the same for a level-3 table
+  __device__ __forceinline__ K level3(K key, K e, uint32_t& r) const {
+    const uint32_t r0 = (uint32_t)(e & 0x7FF), sh = (uint32_t)(e >> 11) & 63u, tb = (uint32_t)(e >> 23) & 63u;
+    const K first = plo[r0 + 1];
+    const K d = (K)(key - first), c = (K)(d >> sh);
+    const uint32_t sub = c < 63 ? (uint32_t)c : 63u;
+    const K soff = d & (K)(((K)1 << sh) - 1);
+    const K e3 = lut[G::L1CELLS + (tb << 6) + sub];
+    const bool below = key < first;
+    r = below ? r0 : (uint32_t)((e3 >> G::S2) & 0x1FFFF) + (soff > (e3 & G::M2) ? 1u : 0u);
+    return below ? (K)0 : e3;
+  }
   // search: the range of key by binary search over the candidates a search
   // entry e names, or over the ranges below / above the window for a key
   // outside it
@@ -1194,7 +1220,8 @@ template <class K> struct Pass0Map {
       if (!out && (e & G::TABLE)) e = level2<WIN>(key, e, r);
       const bool ns = out || (e & G::FLAG) != 0;
       if (wave_ballot(ns)) {
-        if (ns) r = search(key, e, out);
+        if (!out && (e & G::FLAG) && (e & G::DEEP)) e = level3(key, e, r);
+        if (out || (e & G::FLAG)) r = search(key, e, out);
       }
     }
     return r;
@@ -1225,9 +1252,17 @@ template <class K> struct Pass0Map {
         ns |= out[j] || (e[j] & G::FLAG) != 0;
       }
       if (wave_ballot(ns)) {
+        bool far = false;
 #pragma unroll
-        for (int j = 0; j < N; ++j)
-          if (out[j] || (e[j] & G::FLAG)) r[j] = search(key[j], e[j], out[j]);
+        for (int j = 0; j < N; ++j) {
+          if (!out[j] && (e[j] & G::FLAG) && (e[j] & G::DEEP)) e[j] = level3(key[j], e[j], r[j]);
+          far |= out[j] || (e[j] & G::FLAG) != 0;
+        }
+        if (wave_ballot(far)) {
+#pragma unroll
+          for (int j = 0; j < N; ++j)
+            if (out[j] || (e[j] & G::FLAG)) r[j] = search(key[j], e[j], out[j]);
+        }
       }
     }
 #pragma unroll
@@ -1327,16 +1362,43 @@ __device__ uint32_t build_lut(const K* starts, uint32_t R, K* __restrict__ dst, 
   __syncthreads();
   // level 2: 64 sub-cells of each tabled cell
   const uint32_t used = tabs < G::L2TABLES ? tabs : G::L2TABLES;
+  if (used == 0) return 0;
   const uint32_t ssh = wsh - 6;
+  __syncthreads();  // every thread has read it: level 2 takes more
   for (uint32_t i = t; i < used * 64; i += nt) {
     const uint32_t tb = i >> 6, sub = i & 63;
     const K lo = (K)(wbase + ((K)tab_cell[tb] << wsh) + ((K)sub << ssh)), hi = (K)(lo + (((K)1 << ssh) - 1));
     const uint32_t ra = tab_r[tb] & 0xFFFFu, rb = tab_r[tb] >> 16;
     const uint32_t r0 = last_start_le<K>(starts, ra, rb, lo);
     const uint32_t r1 = last_start_le<K>(starts, r0, rb, hi);
+    K e = l2_entry<K>(starts, r0, r1, lo);
+    if (r1 >= r0 + 2) {
+      const K span = (K)(starts[r1] - starts[r0 + 1]);
+      const uint32_t len = bitlen64((uint64_t)span);
+      uint32_t sh = len > 6 ? len - 6 : 0;
+      if ((span >> sh) > 62) ++sh;
+      const uint32_t deep = sh <= G::S2 ? atomicAdd(&tabs, 1u) : G::L2TABLES;
+      if (deep < G::L2TABLES) {
+        tab_cell[deep] = sh;
+        tab_r[deep] = r0 | (r1 << 16);
+        e = G::FLAG | G::DEEP | (K)r0 | ((K)sh << 11) | ((K)deep << 23);
+      }
+    }
+    dst[C + i] = e;
+  }
+  __syncthreads();
+  // level 3: 64 cells from the first start inside each of those sub-cells
+  const uint32_t all = tabs < G::L2TABLES ? tabs : G::L2TABLES;
+  for (uint32_t i = used * 64 + t; i < all * 64; i += nt) {
+    const uint32_t tb = i >> 6, sub = i & 63, sh = tab_cell[tb];
+    const uint32_t ra = (tab_r[tb] & 0xFFFFu) + 1, rb = tab_r[tb] >> 16;
+    const K first = starts[ra], lo = (K)(first + ((K)sub << sh)), hi = (K)(lo + (((K)1 << sh) - 1));
+    const bool past = sub == 63 || lo < first;  // no start there; the key space may end before it
+    const uint32_t r0 = past ? rb : last_start_le<K>(starts, ra, rb, lo);
+    const uint32_t r1 = past || hi < lo ? rb : last_start_le<K>(starts, r0, rb, hi);
     dst[C + i] = l2_entry<K>(starts, r0, r1, lo);
   }
-  return used;
+  return all;
 }
 
 // Plain fill (used instead of hipMemsetAsync so the sequence stays capturable).
@@ -1400,7 +1462,7 @@ __global__ void __launch_bounds__(1024) k_count0(const T* __restrict__ x, const 
   // across the tile boundary; one histogram row per tile
   uint32_t* hist0 = reinterpret_cast<uint32_t*>(smem + Pass0Map<K>::param_bytes(ctl->R));
   for (uint32_t i = threadIdx.x; i < B * tiles_per_wg; i += blockDim.x) hist0[i] = 0;
-  mp.load(lut, ranges, ctl->R);
+  mp.load(lut, ranges, ctl->R, ctl->l2_used);
   mp.set_window(ctl);
   __syncthreads();
   // With a dominant value (its bucket hb), a key of it only adds to a
@@ -2508,7 +2570,7 @@ __global__ void __launch_bounds__(1024) k_compact0(const T* __restrict__ x, cons
   mp.set_params(smem, ctl->R);
   uint16_t* slot = reinterpret_cast<uint16_t*>(smem + Pass0Map<K>::param_bytes(ctl->R));
   for (uint32_t i = threadIdx.x; i < B; i += blockDim.x) slot[i] = slot_of_bucket[i];
-  mp.load(lut, ranges, ctl->R);
+  mp.load(lut, ranges, ctl->R, ctl->l2_used);
   const uint32_t* rp = rows + (size_t)blockIdx.x * B;
   uint32_t acc = 0;
   for (uint32_t s = threadIdx.x; s < U_slots; s += blockDim.x) acc += rp[slot_bucket[s]];
@@ -2694,7 +2756,7 @@ __global__ void __launch_bounds__(1024) k_group_pass0(const T* __restrict__ x,
     s_cnt[1][g] = 0;
     s_run[g] = 0;
   }
-  mp.load(lut, ranges, ctl->R);
+  mp.load(lut, ranges, ctl->R, ctl->l2_used);
   __syncthreads();
   // this tile's survivors per group, from its histogram row: one run per group
   const uint32_t* row = rows + (size_t)blockIdx.x * B;
@@ -2858,7 +2920,7 @@ __global__ void __launch_bounds__(1024) k_group_scatter(const T* __restrict__ x,
   uint16_t* slot = reinterpret_cast<uint16_t*>(smem + Pass0Map<K>::param_bytes(ctl->R));
   for (uint32_t i = t; i < B; i += nt) slot[i] = slot_of_bucket[i];
   for (uint32_t g = t; g < kMaxGroups; g += nt) s_run[g] = 0;
-  mp.load(lut, ranges, ctl->R);
+  mp.load(lut, ranges, ctl->R, ctl->l2_used);
   __syncthreads();
   const uint32_t* row = rows + (size_t)blockIdx.x * B;
   for (uint32_t sl = t; sl < U_slots; sl += nt) {
