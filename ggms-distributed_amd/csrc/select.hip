@@ -164,7 +164,9 @@ static Config resolve_config(ggms_alg alg, uint64_t n, uint32_t nk, const ggms_o
   c.B_cap = kMaxBuckets;
   if (c.mode == kModeLinear || c.mode == kModeStrided) {
     c.P = o.num_pivots ? o.num_pivots : 17;
-    c.P = std::max<uint32_t>(2, std::min<uint32_t>(c.P, 1024));
+    // (950 where the grouped compaction of 4-byte keys holds the ranges'
+    // parameters beside its staging area: 16384 buckets then fit its LDS)
+    c.P = std::max<uint32_t>(2, std::min<uint32_t>(c.P, c.seg_first && sizeof(K) == 4 ? 950 : 1024));
     // the reference's 1024-key sample; a large call with few ks and 4-byte
     // keys draws 2048 (2^28 fp32 N(0,1), 1001 ks: 0.684 -> 0.672 ms, its
     // pieces closer to the quantiles; the many-k calls keep 1024: 2048 is
@@ -404,6 +406,8 @@ constexpr uint32_t kSetupInPlan0MaxKs = kSetupKsPerThread * 1024;
 // LDS ceiling of one workgroup on gfx950 (160 KB per CU; static LDS of the
 // kernels stays under 2 KB).
 constexpr size_t kLdsLimit = 158 * 1024;
+// Tables above this are refused; a kernel's few words of static LDS come on top.
+constexpr size_t kLdsMost = 159 * 1024;
 // dynamic LDS that leaves room for only one 1024-thread workgroup per CU
 constexpr size_t kLdsOneWgPerCu = 81 * 1024;
 
@@ -447,7 +451,7 @@ static void set_lds_attr(const void* fn, size_t bytes) {
 
 #define LDS_CHECK(bytes)                              \
   do {                                                \
-    if ((bytes) > kLdsLimit) return GGMS_ENOTSUP;     \
+    if ((bytes) > kLdsMost) return GGMS_ENOTSUP;      \
   } while (0)
 
 // The plan of a pass of at most B_bound buckets and R_bound ranges: kept in

@@ -30,3 +30,22 @@ def test_exact(dtype, components, sigma, splitter, gpu_ctx):
             got = gpu_ctx.select(x, ks, alg, ggms.default_opts(splitter=splitter, learned_pieces=128 if splitter else 0,
                                                                num_pivots=0 if splitter else 129))
             assert np.array_equal(_bits(got), _bits(want)), (alg, nk)
+
+
+@pytest.mark.parametrize("dtype,pivots", [("float32", 940), ("float32", 985), ("uint32", 1024), ("float64", 500)])
+@pytest.mark.parametrize("nk", [1, 301, 8192, 9000])
+def test_largest_tables(dtype, pivots, nk, gpu_ctx):
+    """the most buckets and many pivots fit every kernel's LDS"""
+    import ggms
+    n = 2_000_003
+    x = ggms.generate(dtype, "uniform" if dtype == "uint32" else "normal", n, 5)
+    order = np.sort(x.cpu().numpy())
+    ks = ggms.generate_ks("even", nk, n, 1)
+    want = order[n - ks.astype(np.int64)]
+    for first_pass in (0, 1, 2):
+        for schedule in (0, 1):
+            o = ggms.default_opts(num_buckets=16384, num_pivots=pivots, sample_size=16384, first_pass=first_pass,
+                                  schedule=schedule)
+            for alg in ("iterative", "bucket"):
+                got = gpu_ctx.select(x, ks, alg, o)
+                assert np.array_equal(_bits(got), _bits(want)), (first_pass, schedule, alg)
