@@ -975,8 +975,9 @@ __device__ __forceinline__ void stream_tile_any(const V* __restrict__ x, uint32_
 // all keys past it), with the entries of level 2.  A search is a read of LDS and
 // a handful of instructions a step for the whole wave, whichever lanes need it:
 // the components of a mixture that are narrow beside their distance from zero
-// put 16 ranges and a tenth of the keys into one sub-cell (2^28 keys, 8192 ks:
-// first-pass count 570 -> 413 us, compaction 1118 -> 955, mean of nine mixtures).
+// put 16 ranges and a tenth of the keys into one sub-cell (2^28 keys, 8192 ks, on
+// such mixtures: first-pass count 590 -> 435 us, compaction 1125 -> 968; the wave-
+// wide test before it costs other inputs' searches 1 us, without one it was 5).
 // The map parameters of a range are packed for one 16-byte (u32 keys) or
 // 32-byte (u64 keys) LDS read.
 // ---------------------------------------------------------------------------
@@ -1000,12 +1001,15 @@ template <class K> struct LutGeom {
   static constexpr uint32_t S1 = KB - L1BITS;
   static constexpr uint32_t S2 = S1 - 6;
   // 10 KB (u32) / 16 KB (u64) of levels 2 and 3.  At 32 the tables of u32 ran
-  // out on one of ten mixtures (2^28 keys 1.87 -> 2.20 ms); 44 and 48 cost the
+  // out on one of ten mixtures (2^28 keys 1.91 -> 2.20 ms); 44 and 48 cost the
   // first-pass count of every input its room in LDS (2^28 N(0,1) 185 -> 191 us).
   static constexpr uint32_t L2TABLES = sizeof(K) == 4 ? 40u : 32u;
   static constexpr K FLAG = (K)1 << (KB - 1);
   static constexpr K TABLE = (K)1 << (KB - 2);
   static constexpr K DEEP = (K)1 << 22;
+  // 4-byte keys only: with 8-byte keys the code alone takes the first-pass
+  // count of 2^27 fp64 N(0,1) from 217 to 225 us
+  static constexpr bool LEVEL3 = sizeof(K) == 4;
   static constexpr K M1 = ((K)1 << S1) - 1;
   static constexpr K M2 = ((K)1 << S2) - 1;
   static __host__ __device__ constexpr size_t bytes() { return (size_t)(L1CELLS + L2TABLES * 64) * sizeof(K); }
@@ -1220,7 +1224,7 @@ template <class K> struct Pass0Map {
       if (!out && (e & G::TABLE)) e = level2<WIN>(key, e, r);
       const bool ns = out || (e & G::FLAG) != 0;
       if (wave_ballot(ns)) {
-        if (!out && (e & G::FLAG) && (e & G::DEEP)) e = level3(key, e, r);
+        if (G::LEVEL3 && !out && (e & G::FLAG) && (e & G::DEEP)) e = level3(key, e, r);
         if (out || (e & G::FLAG)) r = search(key, e, out);
       }
     }
@@ -1252,11 +1256,19 @@ template <class K> struct Pass0Map {
         ns |= out[j] || (e[j] & G::FLAG) != 0;
       }
       if (wave_ballot(ns)) {
-        bool far = false;
+        bool far = ns;
+        if constexpr (G::LEVEL3) {
+          bool deep = false;
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-          if (!out[j] && (e[j] & G::FLAG) && (e[j] & G::DEEP)) e[j] = level3(key[j], e[j], r[j]);
-          far |= out[j] || (e[j] & G::FLAG) != 0;
+          for (int j = 0; j < N; ++j) deep |= !out[j] && (e[j] & (G::FLAG | G::DEEP)) == (G::FLAG | G::DEEP);
+          if (wave_ballot(deep)) {
+            far = false;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+              if (!out[j] && (e[j] & G::FLAG) && (e[j] & G::DEEP)) e[j] = level3(key[j], e[j], r[j]);
+              far |= out[j] || (e[j] & G::FLAG) != 0;
+            }
+          }
         }
         if (wave_ballot(far)) {
 #pragma unroll
@@ -1372,7 +1384,7 @@ __device__ uint32_t build_lut(const K* starts, uint32_t R, K* __restrict__ dst, 
     const uint32_t r0 = last_start_le<K>(starts, ra, rb, lo);
     const uint32_t r1 = last_start_le<K>(starts, r0, rb, hi);
     K e = l2_entry<K>(starts, r0, r1, lo);
-    if (r1 >= r0 + 2) {
+    if (G::LEVEL3 && r1 >= r0 + 2) {
       const K span = (K)(starts[r1] - starts[r0 + 1]);
       const uint32_t len = bitlen64((uint64_t)span);
       uint32_t sh = len > 6 ? len - 6 : 0;
